@@ -67,3 +67,53 @@ def test_qkv_and_gate_up_of_decoded_rows(gpu_ctx, oracle, dtype):
     g, u = W["g"].matmul(x, 1), W["u"].matmul(x, 1)
     exp = (g / (np.float32(1.0) + np.exp(-g))) * u
     assert np.allclose(h, exp, rtol=2e-6, atol=1e-7)
+
+
+# The batched product's three forms (16 x 16 and 32 x 32 blocks with K split
+# over eight waves, 64 x 64 tiles) at ragged rows, batches and widths, and
+# widths or an input address that only single-value loads can read. The bound
+# is the file's: a sum of K f32 terms in any order errs by at most
+# K * 2^-24 * sum|w x|, far below 1e-5 * sum|w x| for these K.
+@pytest.mark.parametrize("dtype,rows,cols,batch,shift", [
+    (F32, 64, 2048, 500, 0), (F16, 17, 129, 33, 0), (F32, 5, 4, 2, 0), (F32, 64, 2048, 64, 1),
+    (F32, 1000, 257, 300, 0), (F16, 1000, 260, 290, 0), (Q8_0, 1100, 96, 257, 0),
+    (F32, 1500, 33, 700, 0), (F16, 1025, 1036, 1000, 0), (F16, 1025, 64, 1000, 1)])
+def test_batched_forms_at_their_edges(gpu_ctx, hyq, oracle, dtype, rows, cols, batch, shift):
+    w = random_matrix(dtype, rows, cols, seed=rows + cols)
+    x = np.random.default_rng(batch).normal(0, 1, batch * cols).astype(np.float32)
+    W = gpu_ctx.upload(dtype, w, (cols, rows))
+    xd = gpu_ctx.array(np.concatenate([np.zeros(shift, np.float32), x]))
+    yd = gpu_ctx.array(np.full(batch * rows + 8, 7.0, np.float32))
+    hyq.check(hyq.lib().hyq_matmul_d(gpu_ctx.handle, W.handle, xd.ptr + 4 * shift, batch, yd.ptr))
+    y = yd.numpy()
+    assert np.all(y[batch * rows:] == 7.0)
+    y = y[:batch * rows].reshape(batch, rows)
+    y_ref, mag = oracle.matmul_f64(dtype, w, rows, cols, x, batch)
+    for b in range(batch):
+        check_decode_path(y[b], y_ref[b], mag[b], f"{dtype} [{rows}x{cols}] b{b}")
+    W.release()
+
+
+@pytest.mark.parametrize("rows,batch", [(64, 40), (1000, 300), (1500, 700)])
+def test_batched_products_keep_small_and_non_finite_values(gpu_ctx, rows, batch):
+    """A column of subnormal weights, an infinity and a NaN in single rows:
+    each only reaches its own outputs."""
+    cols = 96
+    w = np.random.default_rng(1).normal(0, 1, (rows, cols)).astype(np.float32)
+    w[1] = 0
+    w[1, 5] = 1e-39
+    w[2, 3] = np.inf
+    x = np.random.default_rng(2).normal(0, 1, (batch, cols)).astype(np.float32)
+    x[0] = 0
+    x[0, 5] = 1.0
+    x[3, 7] = np.nan
+    W = gpu_ctx.upload(F32, w.view(np.uint8).reshape(-1), (cols, rows))
+    y = W.matmul(x, batch).reshape(batch, rows)
+    assert y[0, 1] == np.float32(1e-39)
+    assert np.isnan(y[3]).all()
+    keep = np.ones((batch, rows), bool)
+    keep[3] = False
+    keep[:, 2] = False
+    assert np.isfinite(y[keep]).all()
+    assert not np.isfinite(y[:, 2]).any()
+    W.release()
