@@ -231,6 +231,56 @@ def test_moe_row_group_streams(gpu_ctx, hyq, oracle, hidden, mid):
               np.stack([mag[t] for t in range(tokens)]), f"row groups {hidden}x{mid}")
 
 
+@pytest.mark.parametrize("tokens,experts,used", [(300, 64, 8), (1024, 64, 8), (4096, 5, 2),
+                                                 (700, 200, 5), (129, 1000, 8)])
+def test_moe_plan_of_many_pairs(gpu_ctx, hyq, oracle, tokens, experts, used):
+    """More pairs than the 1024-pair plan takes, in a random order, with
+    pairs out of range (skipped) and a token routed nowhere: sampled tokens
+    against the f64 chain, and the same call twice (one scratch) bit for bit."""
+    hidden, mid = 256, 256
+    gate = random_matrix(Q4_K, experts * mid, hidden, seed=41)
+    up = random_matrix(Q4_K, experts * mid, hidden, seed=42)
+    down = random_matrix(Q4_K, experts * hidden, mid, seed=43)
+    rng = np.random.default_rng(tokens)
+    x = rng.normal(0, 1, tokens * hidden).astype(np.float32)
+    pt = np.repeat(np.arange(tokens, dtype=np.int32), used)
+    pe = np.concatenate([rng.choice(experts, used, replace=False)
+                         for _ in range(tokens)]).astype(np.int32)
+    pw = rng.uniform(0.1, 1.0, pt.size).astype(np.float32)
+    keep = pt != 17
+    pt, pe, pw = pt[keep], pe[keep], pw[keep]
+    perm = rng.permutation(pt.size)
+    pt, pe, pw = pt[perm], pe[perm], pw[perm]
+    bad = rng.choice(pt.size, 9, replace=False)
+    dt, de = pt.copy(), pe.copy()
+    dt[bad[:3]], dt[bad[3:5]], de[bad[5:7]], de[bad[7:]] = -1, tokens, experts, -5
+    good = np.ones(pt.size, bool)
+    good[bad] = False
+    G = gpu_ctx.upload(Q4_K, gate, (hidden, mid, experts))
+    U = gpu_ctx.upload(Q4_K, up, (hidden, mid, experts))
+    D = gpu_ctx.upload(Q4_K, down, (mid, hidden, experts))
+    L = hyq.lib()
+    nbytes = L.hyq_moe_scratch_bytes(tokens, pt.size, experts, hidden, mid)
+    scratch = gpu_ctx.empty(nbytes, np.uint8)
+    xd, td, ed, wd = (gpu_ctx.array(a) for a in (x, dt, de, pw))
+    outs = []
+    for _ in range(2):
+        od = gpu_ctx.array(np.zeros(tokens * hidden, np.float32))
+        hyq.check(L.hyq_moe_experts_d(gpu_ctx.handle, G.handle, U.handle, D.handle, xd.ptr,
+                                      tokens, td.ptr, ed.ptr, wd.ptr, pt.size, scratch.ptr,
+                                      nbytes, od.ptr))
+        outs.append(od.numpy().reshape(tokens, hidden))
+    assert np.array_equal(outs[0], outs[1])
+    assert not outs[0][17].any()
+    sample = [0, 17, tokens - 1] + [int(t) for t in pt[bad[:2]]] + [int(rng.integers(tokens))]
+    ref, mag = chain_f64(oracle, Q4_K, Q4_K, gate, up, down, hidden, mid, x, pt[good], pe[good],
+                         pw[good], np.zeros((tokens, hidden), np.float32), sample)
+    for t in set(sample) - {17}:
+        check_moe(outs[0][t], ref[t], mag[t], f"token {t}")
+    for w in (G, U, D):
+        w.release()
+
+
 def test_moe_device_entry_point_and_rerun(gpu_ctx, hyq):
     """hyq_moe_experts_d on device buffers equals the host entry point, twice
     in a row on the same scratch (the second with fewer pairs)."""
