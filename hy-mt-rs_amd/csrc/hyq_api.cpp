@@ -474,10 +474,22 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
     if (batch > 65535) return fail(HYQ_EINVAL, "matmul: batch %zu exceeds 65535", batch);
     // Q8_0 at up to 128 tokens: one register-operand launch (no K split)
     const bool few = w->dtype == Q8_0 && few_q80_fits((int)w->rows, (int)w->cols, (int)batch);
-    const int ks = few ? 1 : matmul_kslices(w->dtype, (int)w->rows, (int)w->cols, (int)batch);
-    // the 256-token tiles take their f16 rows in MFMA fragment order
+    // a few tokens: weights dequantized into MFMA operands in registers
+    int ks = 1;
+    bool reg = !few && regmm_fits(w->dtype, (int)w->cols, (int)batch);
+    if (reg) {
+        ks = regmm_kslices((int)w->rows, (int)w->cols);
+        // (both entry points take the same form: only one whose temporaries
+        // fit the fixed array)
+        const size_t need = align_up(frag_rows((int)batch) * w->cols * 2, 256) + batch * 4 +
+                            256 + (ks > 1 ? (size_t)ks * batch * w->rows * 4 : 0);
+        if (need > HYQ_NOALLOC_SCRATCH_BYTES) reg = false;
+    }
+    if (!few && !reg) ks = matmul_kslices(w->dtype, (int)w->rows, (int)w->cols, (int)batch);
+    // these and the 256-token tiles take their f16 rows in MFMA fragment order
     const bool frag =
-        !few && gemm_frag_operand(w->dtype, (int)w->rows, (int)w->cols, (int)batch, ks);
+        reg ||
+        (!few && gemm_frag_operand(w->dtype, (int)w->rows, (int)w->cols, (int)batch, ks));
     const size_t xh_bytes =
         align_up(few ? few_q80_operand_bytes((int)w->cols, (int)batch)
                      : (frag ? frag_rows((int)batch) : batch) * w->cols * 2,
@@ -506,6 +518,12 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
     }
     HYQ_LAUNCH(launch_to_f16(x_d, (int)batch, (int)w->cols, xh, rscale, ctx->stream, frag),
                "to_f16");
+    if (reg) {
+        HYQ_LAUNCH(launch_regmm(w->dtype, w->view, (int)w->cols, xh, rscale, (int)batch, y_d,
+                                nullptr, ctx->stream, ks, (float *)part_mem),
+                   "regmm");
+        return HYQ_OK;
+    }
     HYQ_LAUNCH(launch_gemm_f16(w->dtype, w->view, (int)w->cols, xh, rscale, (int)batch, y_d,
                                nullptr, ctx->stream, (float *)part_mem, part, ks, frag),
                "gemm_f16");

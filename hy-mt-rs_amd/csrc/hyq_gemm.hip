@@ -1244,6 +1244,17 @@ bool gemm_frag_operand(int fmt, int rows, int cols, int batch, int kslices)
     return gemm_waves(batch, mtiles * (kslices > 1 ? kslices : 1)) == 8;
 }
 
+int launch_gemm_reduce(const float *part, int kslices, size_t count, const float *residual,
+                       float *y, void *stream)
+{
+    const size_t count4 = count / 4;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((count4 + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, reinterpret_cast<const float4 *>(part), kslices,
+                       count4, reinterpret_cast<const float4 *>(residual),
+                       reinterpret_cast<float4 *>(y));
+    return (int)hipGetLastError();
+}
+
 int launch_gemm_f16(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale,
                     int batch, float *y, const float *residual, void *stream, float *part,
                     size_t part_floats, int kslices, bool xfrag)
@@ -1258,12 +1269,7 @@ int launch_gemm_f16(int fmt, WView w, int cols, const _Float16 *xh, const float 
     if (ks > 1 && part && part_floats >= (size_t)ks * batch * w.rows) {
         int rc = launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, ks, part, xfrag);
         if (rc) return rc;
-        const size_t count4 = (size_t)batch * w.rows / 4;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((count4 + 255) / 256)), dim3(256),
-                           0, (hipStream_t)stream, reinterpret_cast<const float4 *>(part), ks,
-                           count4, reinterpret_cast<const float4 *>(residual),
-                           reinterpret_cast<float4 *>(y));
-        return (int)hipGetLastError();
+        return launch_gemm_reduce(part, ks, (size_t)batch * w.rows, residual, y, stream);
     }
     return launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, 1, nullptr, xfrag);
 }

@@ -228,6 +228,18 @@ int launch_gemm_f16_segs(int fmt, GemmSegs g, int cols, const _Float16 *xh, cons
                          bool xfrag = false);
 int launch_gate_up_f16(int fmt, WView gate, WView up, int cols, const _Float16 *xh,
                        const float *rscale, int batch, float *h, void *stream);
+// y = residual + (((part[0] + part[1]) + ...) over `count` floats (a multiple
+// of 4, 16-byte aligned): the K slices of a split product in slice order.
+int launch_gemm_reduce(const float *part, int kslices, size_t count, const float *residual,
+                       float *y, void *stream);
+// Few-token products with the weights dequantized into MFMA operands in
+// registers (hyq_regmm.hip) for the shapes of regmm_fits; xh in fragment
+// order (launch_to_f16 with frag). kslices > 1 (regmm_kslices) goes through
+// part [kslices][batch][rows].
+bool regmm_fits(int fmt, int cols, int batch);
+int regmm_kslices(int rows, int cols);
+int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale, int batch,
+                 float *y, const float *residual, void *stream, int kslices, float *part);
 
 // Byte offsets of the MoE scratch regions (hyq_gemm.hip: moe_layout).
 struct MoeLayout {

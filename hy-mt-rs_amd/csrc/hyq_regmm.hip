@@ -1,0 +1,75 @@
+// Which shapes the few-token products of hyq_regmm_impl.hpp take, and their
+// launch by format.
+#include <hip/hip_runtime.h>
+
+#include "hyq_regmm_impl.hpp"
+
+namespace hyq {
+
+extern template int launch_regmm_format<Q2_0C>(const regmm::Args &, int, void *);
+extern template int launch_regmm_format<STQ1_0>(const regmm::Args &, int, void *);
+extern template int launch_regmm_format<Q4_K>(const regmm::Args &, int, void *);
+extern template int launch_regmm_format<Q6_K>(const regmm::Args &, int, void *);
+extern template int launch_regmm_format<Q8_0>(const regmm::Args &, int, void *);
+
+// Up to one or two 32-token blocks, so one workgroup per row tile: past them
+// the weights are dequantized again per 64 tokens and the LDS engine is as
+// fast (Q4_K [14336 x 4096] at 128 tokens 47.7 against 52 us, Q2_0C
+// [2048 x 6144] 33 against 32). Q6_K's second block does not fit the
+// registers (spilled, [4096 x 14336] at 64 tokens 66 against 51 us). At least
+// four 64-column steps per wave: a narrower weight leaves the waves that
+// split its columns without work to overlap.
+bool regmm_fits(int fmt, int cols, int batch)
+{
+    return batch >= 2 && batch <= (fmt == Q6_K ? 32 : 64) && cols % tile::BK == 0 &&
+           cols / tile::BK >= 4 * regmm::WAVES;
+}
+
+// K slices across workgroups, where the row tiles leave CUs without one: to
+// about one workgroup per CU, at least six steps per wave (the sum's launch
+// costs 3.5 us: Q2_0C [2048 x 6144] at 21 tokens 16.4 us in one slice, 14.0
+// in four; [6144 x 2048] 10.0 in one, 12.6 in two). A rule on the weight's
+// shape only, so that a token's result does not depend on the batch.
+int regmm_kslices(int rows, int cols)
+{
+    if (rows % 4) return 1;
+    const int tiles = (rows + 31) / 32, per = cols / tile::BK / regmm::WAVES;
+    int ks = 1;
+    while (ks < 4 && tiles * ks * 2 <= 256 && per / (2 * ks) >= 6) ks *= 2;
+    return ks;
+}
+
+int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale, int batch,
+                 float *y, const float *residual, void *stream, int kslices, float *part)
+{
+    if (!regmm_fits(fmt, cols, batch) || w.rows <= 0 || kslices < 1 || (kslices > 1 && !part))
+        return (int)hipErrorInvalidValue;
+    const int tb = batch > 32 ? 2 : 1;
+    regmm::Args a{};
+    a.g.nseg = 1;
+    a.g.s[0].w = w;
+    a.g.s[0].y = y;
+    a.g.s[0].residual = residual;
+    a.g.s[0].rows = w.rows;
+    a.g.s[0].tiles = a.rtiles = (w.rows + 31) / 32;
+    a.K = cols;
+    a.N = batch;
+    a.groups = (batch + 32 * tb - 1) / (32 * tb);
+    a.kslices = kslices;
+    a.xh = xh;
+    a.rscale = rscale;
+    a.part = part;
+    int rc = (int)hipErrorInvalidValue;
+    switch (fmt) {
+    case Q2_0C: rc = launch_regmm_format<Q2_0C>(a, tb, stream); break;
+    case STQ1_0: rc = launch_regmm_format<STQ1_0>(a, tb, stream); break;
+    case Q4_K: rc = launch_regmm_format<Q4_K>(a, tb, stream); break;
+    case Q6_K: rc = launch_regmm_format<Q6_K>(a, tb, stream); break;
+    case Q8_0: rc = launch_regmm_format<Q8_0>(a, tb, stream); break;
+    default: break;
+    }
+    if (rc || kslices == 1) return rc;
+    return launch_gemm_reduce(part, kslices, (size_t)batch * w.rows, residual, y, stream);
+}
+
+} // namespace hyq

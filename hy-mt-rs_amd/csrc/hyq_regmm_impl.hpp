@@ -1,0 +1,210 @@
+// Batched products of few tokens with the weights dequantized straight into
+// MFMA operands (Weight::matmul at batch 2 .. regmm_max_tokens, src/quant.rs:
+// 272-344, on the f16-MFMA path): no LDS copy of either operand, no barrier
+// in the K loop.
+//
+// Bound. A few tokens leave the matrix cores little to do: the product costs
+// the weights' stream from HBM and each CU's load path - a wave's weight
+// load touches 32 rows' cache lines, and its token fragments (4 KiB per 64
+// columns and 32 tokens) come from L2 for every 32 rows. Timing-only variants
+// at Q4_K [14336 x 4096], 21 tokens (24.9 us with 8 waves): weights read as
+// contiguous KiBs 20.5, no token loads 20.5, both 17.8, no dequantization
+// 23.9. A 128-token tile of the LDS engine (hyq_tile.hpp) spends the same
+// MFMAs on 21 tokens as on 128 and meets a barrier every 64 columns.
+// Measured, with the f16 rows' launch (LDS engine -> this): Q2_0C
+// [6144 x 2048] 21 tokens 17.0 -> 10.1 us, 64 tokens 22.4 -> 12.1; Q4_K
+// [14336 x 4096] 21 tokens 44.5 -> 23.4, 64 tokens 48.5 -> 28.4; Q6_K
+// [4096 x 14336] 21 tokens 46.5 -> 36.1.
+//
+// Form. A workgroup owns 32 weight rows against TB blocks of 32 tokens; its
+// waves split K in 64-column steps, each wave with all of the workgroup's rows
+// and tokens, and meet once, in LDS, where the waves' sums are added in wave
+// order. Lane l of a wave is weight row l % 32 and
+// half h = l / 32 of a step's columns (Deq<F>'s halves): the 32 values it
+// dequantizes are four A fragments of v_mfma_f32_32x32x16_f16 as they are -
+// a 16-deep step may take its columns in any order as long as both operands
+// take the same - so the token fragments, kept in fragment order (8
+// consecutive columns of a token per 16-byte piece), are read at the pieces
+// of those columns. The packed bytes of the next D steps are in registers
+// while one is multiplied.
+//
+// Every weight is the same f16 value as in the LDS engine (one fma
+// bit-identical to the decoder, one rounding); an output's terms are summed
+// in another order. A token's result depends on its own row and the weight's
+// shape only: the same bits at any batch that runs this form.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "hyq_tile.hpp"
+
+#pragma clang fp contract(off)
+
+namespace hyq {
+namespace regmm {
+
+using namespace tile;
+
+// The 8-column piece (of the 64-column step's eight) that fragment i of half
+// h holds, as an offset in halves into the step's fragment-order run: piece g
+// is at (g / 2) * 512 + (g % 2) * 256.
+template <int F> __device__ constexpr int piece(int i, int h)
+{
+    const int c = i < 2 ? Deq<F>::c0(h) + 8 * i : Deq<F>::c1(h) + 8 * (i - 2);
+    return (c / 16) * 512 + (c / 8 % 2) * 256;
+}
+
+// Steps of packed bytes in flight per wave: as many as the registers hold.
+template <int F, int TB> constexpr int depth() { return F == Q6_K || TB > 1 ? 2 : 4; }
+
+// Waves of a workgroup. Four, so that a CU holds up to four workgroups at the
+// 128 registers of a wave and one's loads run under another's products; with
+// 8 and 16 waves Q4_K [14336 x 4096] at 21 tokens took 24.9 and 28.7 us
+// against 23.4.
+constexpr int WAVES = 4;
+
+struct Args {
+    GemmSegs g; // .tiles: row tiles of 32 rows
+    int K, N, groups, rtiles, kslices;
+    const _Float16 *xh; // fragment order
+    const float *rscale;
+    float *part; // [kslices][N][rows] when kslices > 1
+};
+
+template <int F, int TB>
+__global__ __launch_bounds__(64 * WAVES, 4) void regmm_kernel(Args a)
+{
+    using D = Deq<F>;
+    constexpr int DEPTH = depth<F, TB>();
+    __shared__ float4 red[TB][WAVES][4][64];
+    const int total = a.rtiles * a.groups, per = (total + 7) / 8;
+    const int T = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8); // XCD-contiguous
+    if (T >= total || (int)(blockIdx.x / 8) >= per) return;
+    int rt = T / a.groups, sg = 0;
+    const int n0 = (T % a.groups) * (32 * TB);
+    while (sg + 1 < a.g.nseg && rt >= a.g.s[sg].tiles) rt -= a.g.s[sg++].tiles;
+    const GemmSeg &S = a.g.s[sg];
+    const int M = S.rows, K = a.K, N = a.N;
+    const int m0 = rt * 32;
+    const int t = threadIdx.x, lane = t & 63, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+
+    // this wave's steps
+    const int steps = K / BK, z = blockIdx.y;
+    const int z0 = (int)((long)steps * z / a.kslices), z1 = (int)((long)steps * (z + 1) / a.kslices);
+    const int c0 = z0 + (z1 - z0) * wave / WAVES, c1 = z0 + (z1 - z0) * (wave + 1) / WAVES;
+
+    f32x16 acc[TB];
+#pragma unroll
+    for (int f = 0; f < TB; ++f)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[f][e] = 0.f;
+
+    if (c0 < c1) {
+        const RowPtr rp = D::rows(S.w, min(m0 + (lane & 31), M - 1)); // (past the end: unused)
+        const _Float16 *xb[TB];
+        const int nblk = (N + 31) / 32;
+        // piece(i, h) = piece(i, 0) + h * (piece(0, 1) - piece(0, 0))
+        const int hoff = h * (piece<F>(0, 1) - piece<F>(0, 0));
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+            xb[b] = a.xh + (size_t)min(n0 / 32 + b, nblk - 1) * 32 * K + (lane & 31) * 8 + hoff;
+        typename D::Raw raw[DEPTH];
+        half8 B[2][TB][2]; // fragments 0, 1 and 2, 3 of a step
+        auto load_b = [&](int s, int c) {
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    B[s][b][i] = *reinterpret_cast<const half8 *>(xb[b] + (size_t)c * 2048 +
+                                                                  piece<F>(2 * s + i, 0));
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) D::load(raw[d], rp, min(c0 + d, c1 - 1) * BK, h);
+        load_b(0, c0);
+        for (int cb = c0; cb < c1; cb += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                const int c = cb + d;
+                if (c >= c1) break;
+                load_b(1, c);
+                half8 w[4];
+                D::values(raw[d], c & 3, h, w);
+                D::load(raw[d], rp, min(c + DEPTH, c1 - 1) * BK, h);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int b = 0; b < TB; ++b)
+                            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[2 * s + i], B[s][b][i],
+                                                                            acc[b], 0, 0, 0);
+                    if (s == 0) load_b(0, min(c + 1, c1 - 1));
+                }
+            }
+        }
+    }
+
+    // the waves' sums in wave order: a thread takes four rows of one token of
+    // each block
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            red[b][wave][e][lane] = make_float4(acc[b][4 * e], acc[b][4 * e + 1],
+                                                acc[b][4 * e + 2], acc[b][4 * e + 3]);
+    __syncthreads();
+    const int m = m0 + 8 * wave + 4 * h;
+    if (m >= M) return;
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+        const int n = n0 + 32 * b + (lane & 31);
+        if (n >= N) continue;
+        float4 v = red[b][0][wave][lane];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) {
+            const float4 p = red[b][w][wave][lane];
+            v = make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w);
+        }
+        const float sc = a.rscale[n];
+        v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
+        const bool split = a.kslices > 1;
+        float *y = split ? a.part + ((size_t)z * N + n) * M : S.y + (size_t)n * M;
+        const float *rr = !split && S.residual ? S.residual + (size_t)n * M : nullptr;
+        if (m + 3 < M && (M & 3) == 0) {
+            if (rr) {
+                const float4 o = *reinterpret_cast<const float4 *>(rr + m);
+                v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
+            }
+            *reinterpret_cast<float4 *>(y + m) = v;
+        } else {
+            const float e4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (m + e < M) y[m + e] = rr ? rr[m + e] + e4[e] : e4[e];
+        }
+    }
+}
+
+} // namespace regmm
+
+// One format's launches (each format is its own translation unit).
+template <int F> int launch_regmm_format(const regmm::Args &a, int tb, void *stream)
+{
+    const int total = a.rtiles * a.groups;
+    const dim3 grid((total + 7) / 8 * 8, a.kslices), block(64 * regmm::WAVES);
+    hipStream_t st = (hipStream_t)stream;
+    if (tb == 1) {
+        hipLaunchKernelGGL((regmm::regmm_kernel<F, 1>), grid, block, 0, st, a);
+        return (int)hipGetLastError();
+    }
+    if constexpr (F != Q6_K) { // (regmm_fits: one block)
+        if (tb == 2) {
+            hipLaunchKernelGGL((regmm::regmm_kernel<F, 2>), grid, block, 0, st, a);
+            return (int)hipGetLastError();
+        }
+    }
+    return (int)hipErrorInvalidValue;
+}
+
+} // namespace hyq

@@ -48,31 +48,13 @@ __device__ __forceinline__ float h2f(uint32_t bits16)
 
 __device__ __forceinline__ uint32_t byte_of(uint32_t dw, int i) { return (dw >> (8 * i)) & 0xffu; }
 
-// 16 f32 values rounded to f16 (round to nearest even), stored as 32 bytes
-// at a 16-byte aligned LDS address.
-__device__ __forceinline__ void store16(_Float16 *dst, const float (&v)[16])
-{
-    half8 a, b;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const half2v p = __builtin_convertvector((float2v){v[2 * i], v[2 * i + 1]}, half2v);
-        const half2v q = __builtin_convertvector((float2v){v[8 + 2 * i], v[9 + 2 * i]}, half2v);
-        a[2 * i] = p[0];
-        a[2 * i + 1] = p[1];
-        b[2 * i] = q[0];
-        b[2 * i + 1] = q[1];
-    }
-    *reinterpret_cast<half8 *>(dst) = a;
-    *reinterpret_cast<half8 *>(dst + 8) = b;
-}
-
 // ---------------------------------------------------------------------------
 // Per-format dequantization of 32 weights of one row, columns [k0, k0 + 64)
-// half h, to dst (the LDS row, indexed by column offset inside the slice).
-// Which 32 columns a half writes depends on the format; the two halves of a
-// row always cover all 64. load() only issues global loads from the row's
-// plane bases (RowPtr, computed once per thread); convert() does the
-// arithmetic from registers.
+// half h: w[0], w[1] hold the columns c0(h) .. c0(h) + 15 of the slice and
+// w[2], w[3] the columns c1(h) .. c1(h) + 15 (which 32 a half takes depends
+// on the format; the two halves of a row cover all 64). load() only issues
+// global loads from the row's plane bases (RowPtr, computed once per thread);
+// values() does the arithmetic from registers, u = (k0 / 64) % 4.
 //
 // Every value is formed as one fma whose exact result is the decoder's
 // exact value, so the f32 result is bit-identical to decode_unchecked
@@ -95,7 +77,39 @@ __device__ __forceinline__ RowPtr row_ptr(const WView &w, int F_p0, int F_p1, in
 // byte i of x as f32 (v_cvt_f32_ubyte{i})
 __device__ __forceinline__ float ub(uint32_t x, int i) { return (float)((x >> (8 * i)) & 0xffu); }
 
+// Eight codes (the bytes of lo, then of hi) as f16(d * q + o).
+__device__ __forceinline__ half8 deq8(uint32_t lo, uint32_t hi, float d, float o)
+{
+    half8 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t x = i < 2 ? lo : hi;
+        const int j = 2 * (i & 1);
+        const half2v p = __builtin_convertvector((float2v){__builtin_fmaf(d, ub(x, j), o),
+                                                           __builtin_fmaf(d, ub(x, j + 1), o)},
+                                                 half2v);
+        r[2 * i] = p[0];
+        r[2 * i + 1] = p[1];
+    }
+    return r;
+}
+
 template <int F> struct Deq;
+
+// The values rounded to f16 at their columns of dst (an LDS row).
+template <int F>
+__device__ __forceinline__ void convert(const typename Deq<F>::Raw &r, int u, int h,
+                                        _Float16 *dst)
+{
+    half8 w[4];
+    Deq<F>::values(r, u, h, w);
+    half8 *p0 = reinterpret_cast<half8 *>(dst + Deq<F>::c0(h));
+    half8 *p1 = reinterpret_cast<half8 *>(dst + Deq<F>::c1(h));
+    p0[0] = w[0];
+    p0[1] = w[1];
+    p1[0] = w[2];
+    p1[1] = w[3];
+}
 
 // Q4_K (decode_unchecked, src/quant.rs:2437-2461): byte l of a 64-weight
 // chunk holds weight l (low nibble, sub-block 2c) and 32 + l (high nibble,
@@ -105,6 +119,8 @@ template <> struct Deq<Q4_K> {
     struct Raw {
         uint4 q, meta;
     };
+    __device__ static constexpr int c0(int h) { return 16 * h; }
+    __device__ static constexpr int c1(int h) { return 32 + 16 * h; }
     __device__ __forceinline__ static RowPtr rows(const WView &w, int row)
     {
         return row_ptr(w, 128, 16, 0, row);
@@ -129,28 +145,22 @@ template <> struct Deq<Q4_K> {
             m = (sc(j + 4) >> 4) | ((sc(j) >> 6) << 4);
         }
     }
-    __device__ __forceinline__ static void convert(const Raw &r, int u, int h, _Float16 *dst)
+    __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
         const int c = u;
         const float d = h2f(r.meta.x & 0xffffu), dmin = h2f(r.meta.x >> 16);
         int s0, m0, s1, m1;
         scale_min(r.meta, 2 * c, s0, m0);
         scale_min(r.meta, 2 * c + 1, s1, m1);
-        const float d1a = d * (float)s0, nm1a = -(dmin * (float)m0);
-        const float d1b = d * (float)s1, nm1b = -(dmin * (float)m1);
+        const float da = d * (float)s0, nm1a = -(dmin * (float)m0);
+        const float db = d * (float)s1, nm1b = -(dmin * (float)m1);
         const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
-        float lo[16], hi[16];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t l = q[w] & 0x0F0F0F0Fu, u = (q[w] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lo[4 * w + i] = __builtin_fmaf(d1a, ub(l, i), nm1a);
-                hi[4 * w + i] = __builtin_fmaf(d1b, ub(u, i), nm1b);
-            }
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t x = q[2 * i], y = q[2 * i + 1];
+            w[i] = deq8(x & 0x0F0F0F0Fu, y & 0x0F0F0F0Fu, da, nm1a);
+            w[2 + i] = deq8((x >> 4) & 0x0F0F0F0Fu, (y >> 4) & 0x0F0F0F0Fu, db, nm1b);
         }
-        store16(dst + 16 * h, lo);
-        store16(dst + 32 + 16 * h, hi);
     }
 };
 
@@ -163,6 +173,8 @@ template <> struct Deq<Q6_K> {
         uint4 l0, l1, g0, g1;
         uint32_t sc, d;
     };
+    __device__ static constexpr int c0(int h) { return 32 * h; }
+    __device__ static constexpr int c1(int h) { return 32 * h + 16; }
     __device__ __forceinline__ static RowPtr rows(const WView &w, int row)
     {
         return row_ptr(w, 192, 16, 2, row);
@@ -179,7 +191,7 @@ template <> struct Deq<Q6_K> {
         r.sc = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 16 + chunk * 8 + 2 * pl);
         r.d = *reinterpret_cast<const uint16_t *>(p.p2 + blk * 2);
     }
-    __device__ __forceinline__ static void convert(const Raw &r, int u, int h, _Float16 *dst)
+    __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
         const int pl = 2 * (u & 1) + h;
         const float d = h2f(r.d);
@@ -188,20 +200,14 @@ template <> struct Deq<Q6_K> {
         const uint32_t ql[8] = {r.l0.x, r.l0.y, r.l0.z, r.l0.w, r.l1.x, r.l1.y, r.l1.z, r.l1.w};
         const uint32_t qh[8] = {r.g0.x, r.g0.y, r.g0.z, r.g0.w, r.g1.x, r.g1.y, r.g1.z, r.g1.w};
         const int lsh = (pl >> 1) * 4, hsh = 2 * pl;
-        float v0[16], v1[16];
+        auto codes = [&](int i) {
+            return ((ql[i] >> lsh) & 0x0F0F0F0Fu) | (((qh[i] >> hsh) & 0x03030303u) << 4);
+        };
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t qa = ((ql[w] >> lsh) & 0x0F0F0F0Fu) | (((qh[w] >> hsh) & 0x03030303u) << 4);
-            const uint32_t qb =
-                ((ql[4 + w] >> lsh) & 0x0F0F0F0Fu) | (((qh[4 + w] >> hsh) & 0x03030303u) << 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v0[4 * w + i] = __builtin_fmaf(s0, ub(qa, i), o0);
-                v1[4 * w + i] = __builtin_fmaf(s1, ub(qb, i), o1);
-            }
+        for (int i = 0; i < 2; ++i) {
+            w[i] = deq8(codes(2 * i), codes(2 * i + 1), s0, o0);
+            w[2 + i] = deq8(codes(4 + 2 * i), codes(5 + 2 * i), s1, o1);
         }
-        store16(dst + 32 * h, v0);
-        store16(dst + 32 * h + 16, v1);
     }
 };
 
@@ -211,6 +217,8 @@ template <> struct Deq<Q8_0> {
         uint4 a, b;
         uint32_t d;
     };
+    __device__ static constexpr int c0(int h) { return 32 * h; }
+    __device__ static constexpr int c1(int h) { return 32 * h + 16; }
     __device__ __forceinline__ static RowPtr rows(const WView &w, int row)
     {
         return row_ptr(w, 32, 2, 0, row);
@@ -222,22 +230,13 @@ template <> struct Deq<Q8_0> {
         r.b = *reinterpret_cast<const uint4 *>(p.p0 + blk * 32 + 16);
         r.d = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 2);
     }
-    __device__ __forceinline__ static void convert(const Raw &r, int, int h, _Float16 *dst)
+    __device__ __forceinline__ static void values(const Raw &r, int, int h, half8 (&w)[4])
     {
         const float d = h2f(r.d), o = -128.f * d;
         const uint32_t q[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
-        float v0[16], v1[16];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t qa = q[w] ^ 0x80808080u, qb = q[4 + w] ^ 0x80808080u; // q + 128
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v0[4 * w + i] = __builtin_fmaf(d, ub(qa, i), o);
-                v1[4 * w + i] = __builtin_fmaf(d, ub(qb, i), o);
-            }
-        }
-        store16(dst + 32 * h, v0);
-        store16(dst + 32 * h + 16, v1);
+        for (int i = 0; i < 4; ++i) // q + 128
+            w[i] = deq8(q[2 * i] ^ 0x80808080u, q[2 * i + 1] ^ 0x80808080u, d, o);
     }
 };
 
@@ -249,6 +248,8 @@ template <> struct Deq<Q2_0C> {
         uint4 c;
         uint32_t d;
     };
+    __device__ static constexpr int c0(int h) { return 32 * h; }
+    __device__ static constexpr int c1(int h) { return 32 * h + 16; }
     __device__ __forceinline__ static RowPtr rows(const WView &w, int row)
     {
         return row_ptr(w, 128, 2, 0, row);
@@ -259,23 +260,16 @@ template <> struct Deq<Q2_0C> {
         r.c = *reinterpret_cast<const uint4 *>(p.p0 + blk * 128 + u * 16);
         r.d = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 2);
     }
-    __device__ __forceinline__ static void convert(const Raw &r, int, int h, _Float16 *dst)
+    __device__ __forceinline__ static void values(const Raw &r, int, int h, half8 (&w)[4])
     {
         const float d = h2f(r.d), d2 = 2.f * d, o = -3.f * d;
         const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
-        float v0[16], v1[16];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t x0 = (cw[w] >> (4 * h)) & 0x03030303u;
-            const uint32_t x1 = (cw[w] >> (4 * h + 2)) & 0x03030303u;
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v0[4 * w + i] = __builtin_fmaf(d2, ub(x0, i), o);
-                v1[4 * w + i] = __builtin_fmaf(d2, ub(x1, i), o);
-            }
-        }
-        store16(dst + 32 * h, v0);
-        store16(dst + 32 * h + 16, v1);
+            for (int k = 0; k < 2; ++k)
+                w[2 * k + i] = deq8((cw[2 * i] >> (4 * h + 2 * k)) & 0x03030303u,
+                                    (cw[2 * i + 1] >> (4 * h + 2 * k)) & 0x03030303u, d2, o);
     }
 };
 
@@ -290,6 +284,8 @@ template <> struct Deq<STQ1_0> {
         uint2 nib;
         uint32_t s, d;
     };
+    __device__ static constexpr int c0(int h) { return 32 * h; }
+    __device__ static constexpr int c1(int h) { return 32 * h + 16; }
     __device__ __forceinline__ static RowPtr rows(const WView &w, int row)
     {
         return row_ptr(w, 32, 8, 2, row);
@@ -301,27 +297,24 @@ template <> struct Deq<STQ1_0> {
         r.s = *reinterpret_cast<const uint32_t *>(p.p1 + blk * 8 + 4 * (c >> 1));
         r.d = *reinterpret_cast<const uint16_t *>(p.p2 + blk * 2);
     }
-    __device__ __forceinline__ static void convert(const Raw &r, int u, int h, _Float16 *dst)
+    __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
         const int c = u;
         const float d = h2f(r.d), o = -d;
         const uint32_t nb[2] = {r.nib.x, r.nib.y};
-        float v0[16], v1[16];
+        uint32_t e[4]; // the groups' codebook entries, four per dword
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t nibs = (nb[j >> 1] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
             const uint32_t sb = ((r.s >> ((c & 1) * 4 + j)) & 0x01010101u) << 4;
-            const uint32_t e = GroupSTQ::lut(nibs | sb);
-            const uint32_t da = (e >> (4 * h)) & 0x03030303u;
-            const uint32_t db = (e >> (4 * h + 2)) & 0x03030303u;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v0[4 * j + i] = __builtin_fmaf(d, ub(da, i), o);
-                v1[4 * j + i] = __builtin_fmaf(d, ub(db, i), o);
-            }
+            e[j] = GroupSTQ::lut(nibs | sb) >> (4 * h);
         }
-        store16(dst + 32 * h, v0);
-        store16(dst + 32 * h + 16, v1);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                w[2 * k + i] = deq8((e[2 * i] >> (2 * k)) & 0x03030303u,
+                                    (e[2 * i + 1] >> (2 * k)) & 0x03030303u, d, o);
     }
 };
 
@@ -455,7 +448,7 @@ __device__ __forceinline__ void k_loop(const WSrc &wsrc, const XRow &xrow, const
     auto put = [&](int k0, int b) {
         _Float16 *Ws = lds + b * BUF;
         if (wthr) {
-            if (row >= 0) D::convert(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
+            if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
             else zero_half(Ws + lrow * LDK, h);
         }
         store_x<NW>(Ws + TILE_HALVES, xr);
@@ -558,7 +551,7 @@ __device__ __forceinline__ void k_loop_pc(const WSrc &wsrc, const XRow &xrow, co
     };
     auto put_w = [&](int k0, int b) {
         _Float16 *Ws = lds + b * BUF;
-        if (row >= 0) D::convert(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
+        if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
         else zero_half(Ws + lrow * LDK, h);
     };
     // Two loops, one per role, each passing the same 1 + steps barriers (a
@@ -639,7 +632,7 @@ __device__ __forceinline__ void k_loop_pcx(const WSrc &wsrc, const XSrc &xsrc, i
         };
         auto put = [&](int k0, int b) {
             _Float16 *Ws = lds + b * TILE_HALVES + lrow * LDK;
-            if (row >= 0) D::convert(raw, ((kbase + k0) >> 6) & 3, h, Ws);
+            if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws);
             else if (used) zero_half(Ws, h);
         };
         fetch(0);

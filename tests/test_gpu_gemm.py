@@ -221,3 +221,37 @@ def test_f16_range_of_batched_weights(gpu_ctx):
             with pytest.raises(ValueError, match="f16"):
                 W.matmul(x, 2)
         W.release()
+
+
+# The register-operand products (2..64 tokens; Q6_K 2..32): one and two token
+# blocks at their edges, row counts that end inside a 32-row tile, four to
+# many 64-column steps per wave shared unevenly, K slices across workgroups
+# ([.. x 6144] and wider at few rows). Bound as the file states it.
+@pytest.mark.parametrize("dtype,rows,cols", [(Q2_0C, 200, 1024), (Q2_0C, 64, 6144),
+                                             (STQ1_0, 33, 1280), (STQ1_0, 132, 7168),
+                                             (Q4_K, 31, 1024), (Q4_K, 1000, 4352),
+                                             (Q6_K, 97, 1536), (Q6_K, 256, 14336),
+                                             (Q8_0, 70, 1088), (Q8_0, 36, 6208)],
+                         ids=lambda v: NAMES.get(v, str(v)))
+def test_register_operand_products(gpu_ctx, hyq, oracle, dtype, rows, cols):
+    w = random_matrix(dtype, rows, cols, seed=rows + cols)
+    W = gpu_ctx.upload(dtype, w, (cols, rows))
+    top = 32 if dtype == Q6_K else 64
+    x = np.random.default_rng(rows).normal(0, 1, top * cols).astype(np.float32)
+    x[cols:2 * cols] *= 1e6  # (the row scales)
+    full = W.matmul(x, top).reshape(top, rows)
+    y_ref, mag = oracle.matmul_f64(dtype, w, rows, cols, x, top)
+    check_prefill_path(full, y_ref, mag, f"{NAMES[dtype]} [{rows}x{cols}]")
+    xd = gpu_ctx.array(x)
+    yd = gpu_ctx.array(np.full(top * rows + 16, 5.0, np.float32))
+    for batch in (2, 17, 31, 32, 33, 63):
+        if batch > top:
+            continue
+        part = W.matmul(x[:batch * cols], batch).reshape(batch, rows)
+        assert np.array_equal(part, full[:batch]), batch  # a row's bits at any batch
+    for fn in (hyq.lib().hyq_matmul_d, hyq.lib().hyq_matmul_noalloc_d):
+        hyq.check(fn(gpu_ctx.handle, W.handle, xd.ptr, top, yd.ptr))
+        y = yd.numpy()
+        assert np.array_equal(y[:top * rows].reshape(top, rows), full)
+        assert np.all(y[top * rows:] == 5.0)
+    W.release()
