@@ -481,18 +481,14 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
         ks = regmm_kslices((int)w->rows, (int)w->cols);
         // (both entry points take the same form: only one whose temporaries
         // fit the fixed array)
-        const size_t need = align_up(frag_rows((int)batch) * w->cols * 2, 256) + batch * 4 +
+        const size_t need = align_up(batch * w->cols * 2, 256) + batch * 4 +
                             256 + (ks > 1 ? (size_t)ks * batch * w->rows * 4 : 0);
         if (need > HYQ_NOALLOC_SCRATCH_BYTES) reg = false;
     }
     if (!few && !reg) ks = matmul_kslices(w->dtype, (int)w->rows, (int)w->cols, (int)batch);
-    // these and the 256-token tiles take their f16 rows in MFMA fragment order
-    const bool frag =
-        reg ||
-        (!few && gemm_frag_operand(w->dtype, (int)w->rows, (int)w->cols, (int)batch, ks));
     const size_t xh_bytes =
         align_up(few ? few_q80_operand_bytes((int)w->cols, (int)batch)
-                     : (frag ? frag_rows((int)batch) : batch) * w->cols * 2,
+                     : batch * w->cols * 2,
                  256);
     const size_t part = ks > 1 ? (size_t)ks * batch * w->rows : 0;
     void *xh_mem = nullptr, *part_mem = nullptr;
@@ -516,7 +512,7 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
                    "few_q80");
         return HYQ_OK;
     }
-    HYQ_LAUNCH(launch_to_f16(x_d, (int)batch, (int)w->cols, xh, rscale, ctx->stream, frag),
+    HYQ_LAUNCH(launch_to_f16(x_d, (int)batch, (int)w->cols, xh, rscale, ctx->stream),
                "to_f16");
     if (reg) {
         HYQ_LAUNCH(launch_regmm(w->dtype, w->view, (int)w->cols, xh, rscale, (int)batch, y_d,
@@ -525,7 +521,7 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
         return HYQ_OK;
     }
     HYQ_LAUNCH(launch_gemm_f16(w->dtype, w->view, (int)w->cols, xh, rscale, (int)batch, y_d,
-                               nullptr, ctx->stream, (float *)part_mem, part, ks, frag),
+                               nullptr, ctx->stream, (float *)part_mem, part, ks),
                "gemm_f16");
     return HYQ_OK;
 }

@@ -271,9 +271,9 @@ __global__ __launch_bounds__(256, 2) void attn_rows_kernel(
 // tokens, 256 threads), reading only the splits the token sees (splits
 // 0 .. (pos + chunk) / chunk - 1): per head M = max_s m_s, w_s =
 // exp(m_s - M), row = (sum_s w_s acc_s) / (sum_s w_s l_s), sums in split
-// order. It writes the f32 row to out (if given) and/or the row as f16 with
-// its power-of-two scale (xh, rscale: the attention-output GEMM's operand,
-// rows_to_f16_kernel's rounding). Dynamic LDS: the row (heads * 128 floats)
+// order. It writes the f32 row to out (if given) and/or the row as f16 in
+// fragment order with its power-of-two scale (xh, rscale: the attention-output
+// GEMM's operand, rows_to_f16_kernel's rounding). Dynamic LDS: the row (heads * 128 floats)
 // and the per-(head, split) weights (heads * splits floats, twice).
 __global__ __launch_bounds__(256) void merge_rows_kernel(const float *__restrict__ part,
                                                          int splits, int chunk, int heads,
@@ -325,7 +325,9 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const float *__restrict
     const int e = f16_row_exponent(mx);
     const float inv = ldexpf(1.0f, -e);
     if (t == 0) rscale[tq] = ldexpf(1.0f, e);
-    for (int i = t; i < W; i += 256) xh[(size_t)tq * W + i] = (_Float16)(row[i] * inv);
+    const int first = tq & ~31, bt = min(32, (int)gridDim.x - first);
+    _Float16 *o = xh + (size_t)first * W;
+    for (int i = t; i < W; i += 256) o[frag_at(i, tq - first, bt)] = (_Float16)(row[i] * inv);
 }
 
 } // namespace

@@ -21,6 +21,17 @@ __device__ __forceinline__ int f16_row_exponent(float m)
     return e;
 }
 
+// The fragment order of a batched product's f16 operand: 32-token blocks, one
+// after the other, each as the B operands of v_mfma_f32_32x32x16_f16 take it -
+// column k of the block's token t at (k / 16) * 16 c + (k / 8 % 2) * 8 c +
+// 8 t + k % 8 halves for a block of c tokens (32, or what is left), so 8
+// consecutive columns of a token are one 16-byte piece, a full block's
+// fragment is one contiguous KiB, and n rows take n * K halves.
+__device__ __forceinline__ size_t frag_at(int k, int t, int c)
+{
+    return (size_t)(k / 8) * 8 * c + 8 * t + k % 8;
+}
+
 // The token row of workgroup b when the rows are written in an MFMA
 // fragment order whose 128-byte lines hold 16 bytes of each of 8
 // consecutive rows (r / 8 equal), and workgroup b runs on XCD b % 8: with row

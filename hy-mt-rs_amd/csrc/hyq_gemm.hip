@@ -6,14 +6,15 @@
 //                 gate/up GEMM with the SiLU product in its epilogue and a
 //                 down GEMM, then the routed sum in ascending expert order.
 //
-// Activations are rounded to f16 once (to_f16 / the gate-up epilogue) and
-// read by the tiles as f16. Tile order is XCD-aware: workgroups are
+// Activations are rounded to f16 once, into the fragment order of
+// hyq_f16rows.hpp, and read by the tiles as f16. Tile order is XCD-aware: workgroups are
 // dispatched round-robin over the 8 XCDs, so workgroup b runs on XCD b % 8;
 // tile (b % 8) * per + b / 8 gives each XCD a contiguous range of tiles, and
 // the tiles sharing one weight row block land on the same XCD and its L2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "hyq_f16rows.hpp"
 #include "hyq_few_q80.hpp"
@@ -42,8 +43,10 @@ __device__ __forceinline__ int xcd_tile(int total)
 // e = ceil(log2(max_k |v[k]|)) - 14 puts the row's largest magnitude at or
 // below 2^14, so no value overflows f16 or drops into its subnormals; the
 // power-of-two scale is exact and the GEMM epilogues multiply it back.
-// src = r, or ptok[order[r]] when order is given; rows r >= *count (when
-// count is given) are left alone. A row with a zero, infinite or NaN maximum
+// src = r, or ptok[order[r]] when ptok is given; rows r >= *count (when
+// count is given) are left alone. xh is in fragment order (hyq_f16rows.hpp):
+// the rows' 32-token blocks, or those of each expert's rows (expert
+// pexp[order[r]] at rows eoff[e] ..) when pexp is given. A row with a zero, infinite or NaN maximum
 // keeps scale 1 (and its infinities / NaNs propagate).
 //
 // R > 0 (rows of at most 1024 R values): thread t holds float4s t + 256 j,
@@ -63,12 +66,22 @@ __global__ __launch_bounds__(256) void rows_to_f16_kernel(const float *__restric
                                                           float eps,
                                                           _Float16 *__restrict__ xh,
                                                           float *__restrict__ rscale,
-                                                          bool frag)
+                                                          const int *__restrict__ pexp,
+                                                          const int *__restrict__ eoff)
 {
     __shared__ float wred[4];
-    const int r = frag ? frag_row((int)blockIdx.x) : (int)blockIdx.x;
+    const int r = frag_row((int)blockIdx.x);
     if (r >= nrows || (count && r >= *count)) return;
-    const size_t src = order ? (size_t)ptok[order[r]] : (size_t)r;
+    const size_t src = ptok ? (size_t)ptok[order[r]] : (size_t)r;
+    // the row's 32-token block: of all rows, or of its expert's rows
+    int first = 0, end = nrows;
+    if (pexp) {
+        const int ex = pexp[order[r]];
+        first = eoff[ex];
+        end = eoff[ex + 1];
+    }
+    first += (r - first) & ~31;
+    const int bt = min(32, end - first);
     const float4 *x4 = reinterpret_cast<const float4 *>(x + src * K);
     const float4 *n4p = reinterpret_cast<const float4 *>(norm);
     const int t = threadIdx.x, n4 = K / 4;
@@ -134,31 +147,31 @@ __global__ __launch_bounds__(256) void rows_to_f16_kernel(const float *__restric
     const int e = f16_row_exponent(m);
     const float inv = ldexpf(1.0f, -e);
     if (t == 0) rscale[r] = ldexpf(1.0f, e);
-    // (fragment order: values 4i .. 4i + 3 stay together, k % 8 being 0 or 4)
-    _Float16 *o = frag ? xh + (size_t)(r / 32) * 32 * K + (size_t)(r % 32) * 8 : xh + (size_t)r * K;
+    // (values 4i .. 4i + 3 stay together, k % 8 being 0 or 4)
+    _Float16 *o = xh + (size_t)first * K;
     each([&](int j, int i) {
         const float4 v = value(j, i);
         const half2v a = __builtin_convertvector((float2v){v.x * inv, v.y * inv}, half2v);
         const half2v b = __builtin_convertvector((float2v){v.z * inv, v.w * inv}, half2v);
-        const int k = 4 * i;
-        _Float16 *q = frag ? o + (size_t)(k / 16) * 512 + 256 * ((k / 8) & 1) + (k & 4) : o + k;
+        _Float16 *q = o + frag_at(4 * i, r - first, bt);
         *reinterpret_cast<half2v *>(q) = a;
         *reinterpret_cast<half2v *>(q + 2) = b;
     });
 }
 
 // rows_to_f16_kernel for rows of K values: the register form with the fewest
-// registers that holds the row, else the loop. In fragment order the grid
-// is the rows rounded up to 64 (see frag_row).
+// registers that holds the row, else the loop. The grid is the rows rounded
+// up to 64 (see frag_row).
 void launch_rows_to_f16(int rows, int K, hipStream_t st, const float *x, const int *order,
                         const int *ptok, const int *count, const float *norm, float eps,
-                        _Float16 *xh, float *rscale, bool frag)
+                        _Float16 *xh, float *rscale, const int *pexp = nullptr,
+                        const int *eoff = nullptr)
 {
     const int need = K < 4 ? 1 << 30 : (K + 1023) / 1024;
-    const dim3 grid(frag ? (rows + 63) / 64 * 64 : rows);
+    const dim3 grid((rows + 63) / 64 * 64);
 #define HYQ_ROWS_F16(RR)                                                                       \
     hipLaunchKernelGGL(rows_to_f16_kernel<RR>, grid, dim3(256), 0, st, x, K, rows, order, ptok, \
-                       count, norm, eps, xh, rscale, frag)
+                       count, norm, eps, xh, rscale, pexp, eoff)
     if (need <= 2) HYQ_ROWS_F16(2);
     else if (need <= 4) HYQ_ROWS_F16(4);
     else if (need <= 6) HYQ_ROWS_F16(6);
@@ -169,52 +182,84 @@ void launch_rows_to_f16(int rows, int K, hipStream_t st, const float *x, const i
 #undef HYQ_ROWS_F16
 }
 
+// The tile shapes of k_loop_px, with the waves per SIMD their registers leave.
+// Tile128 and Tile64 run two workgroups on a CU. Forms with eight producer waves (8 + 8
+// waves of 2 x 2 blocks for 256 tokens, 8 + 4 for 128), against the one
+// instruction per 8 cycles that a SIMD issues for a single wave, measured the
+// same or slower: with MFMAs on all CUs the clock, set by the power drawn, is
+// what the producers' waits would hide under.
+struct Tile256 { // 128 rows x 256 tokens
+    static constexpr int NP = 4, NC = 4, WR = 1, RB = 4, CB = 2, NS = 2, OCC = 2;
+};
+struct Tile256R96 { // 96 rows x 256 tokens
+    static constexpr int NP = 4, NC = 4, WR = 1, RB = 3, CB = 2, NS = 2, OCC = 2;
+};
+struct Tile192 { // 128 rows x 192 tokens
+    static constexpr int NP = 4, NC = 4, WR = 2, RB = 2, CB = 3, NS = 2, OCC = 2;
+};
+struct Tile128 { // 128 rows x 128 tokens
+    static constexpr int NP = 4, NC = 4, WR = 2, RB = 2, CB = 2, NS = 1, OCC = 4;
+};
+struct Tile64 { // 64 rows x 256 tokens
+    static constexpr int NP = 4, NC = 4, WR = 1, RB = 2, CB = 2, NS = 1, OCC = 4;
+};
+using TileMoe = Tile128; // an expert's chunk: BN tokens
+template <class C> constexpr int tile_tokens() { return 32 * (C::NC / C::WR) * C::CB; }
+template <class C> constexpr int tile_rows() { return 32 * C::WR * C::RB; }
+template <class C> constexpr int tile_threads() { return 64 * (C::NP + C::NC); }
+template <class C> __device__ __forceinline__ int px_wr()
+{
+    return ((int)(threadIdx.x >> 6) - C::NP) / (C::NC / C::WR);
+}
+// token of the tile that this lane's column of block j holds
+template <class C> __device__ __forceinline__ int px_token(int j)
+{
+    constexpr int WC = C::NC / C::WR;
+    return 32 * (j * WC + ((int)(threadIdx.x >> 6) - C::NP) % WC) + (threadIdx.x & 31);
+}
+
 // Y[n][m] = (X[n] . W[m]) * rscale[n], plus residual[n][m] when given (the
 // residual add of src/model.rs:595, 601 after the product is rounded; it
 // may alias y: each element is read and then written by one thread). The
 // row space is up to three weights sharing the activation rows (Q, K and V
-// in one launch); a tile's BM rows lie in one of them (its row count is a
+// in one launch); a tile's rows lie in one of them (its row count is a
 // multiple of BM, or it is the last). With kslices > 1 (one weight) grid.y
 // splits K: slice z writes its scaled partial product to
-// part[z][n][m] and gemm_reduce_kernel adds the slices in order. NW waves
-// per workgroup: tiles of BM rows by 32 NW tokens, the same arithmetic per
-// element for NW = 4 and 8 (the 256-token tiles of a plain product run as
-// gemm_f16_pc_kernel, the same arithmetic again).
-template <int F, int NW>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_f16_kernel(
+// part[z][n][m] and gemm_reduce_kernel adds the slices in order.
+template <int F, class C>
+__global__ __launch_bounds__(tile_threads<C>(), C::OCC) void gemm_f16_kernel(
     GemmSegs g, int K, const _Float16 *__restrict__ xh, const float *__restrict__ rscale, int N,
     int mtiles, int ntiles, int kslices, float *__restrict__ part)
 {
-    __shared__ __attribute__((aligned(16))) _Float16 lds[lds_halves<NW>()];
+    __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
     const int T = xcd_tile(mtiles * ntiles);
     if (T >= mtiles * ntiles) return;
     int mt = T / ntiles, sg = 0;
     while (sg + 1 < g.nseg && mt >= g.s[sg].tiles) mt -= g.s[sg++].tiles;
     const GemmSeg &S = g.s[sg];
     const int M = S.rows;
-    const int m0 = mt * BM, n0 = (T % ntiles) * (32 * NW);
-    const int wave = threadIdx.x >> 6, wm = wave / (NW / 2), wn = wave % (NW / 2);
+    const int m0 = mt * tile_rows<C>(), n0 = (T % ntiles) * tile_tokens<C>();
+    const int wr = px_wr<C>();
 
-    f32x16 acc[2][2];
-    zero_acc(acc);
+    f32x16 acc[C::RB][C::CB];
     auto wsrc = [&](int lrow, WView &v, int &row) {
         v = S.w;
-        row = m0 + lrow < M ? m0 + lrow : -1;
+        row = min(m0 + lrow, M - 1);
     };
-    auto xrow = [&](int r) -> const _Float16 * {
-        return n0 + r < N ? xh + (size_t)(n0 + r) * K : nullptr;
-    };
-    auto arow = [&](int i) { return wm * 64 + 32 * i; };
+    auto arow = [&](int i) { return 32 * (wr * C::RB + i); };
     const int kslice = K / kslices;
-    k_loop<F, 2, NW>(wsrc, xrow, arow, kslice, wn, lds, acc, blockIdx.y * kslice);
+    if (!k_loop_px<F, C>(wsrc, arow, xh + (size_t)n0 * K,
+                                                  min(tile_tokens<C>(), N - n0), K,
+                                                  blockIdx.y * kslice, kslice, lds, acc))
+        return;
 
     float *y = kslices > 1 ? part + (size_t)blockIdx.y * N * M : S.y;
     const float *residual = kslices > 1 ? nullptr : S.residual;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < C::RB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + acc_col(wn, j);
+        for (int j = 0; j < C::CB; ++j) {
+            const int n = n0 + px_token<C>(j);
             if (n >= N) continue;
             float *yr = y + (size_t)n * M;
             const float *rr = residual ? residual + (size_t)n * M : nullptr;
@@ -222,153 +267,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_f16_kernel(
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int m = m0 + arow(i) + acc_row_in_block(4 * g4);
-                if (m + 3 < M && (M & 3) == 0) {
-                    float4 v = make_float4(acc[i][j][4 * g4] * sc, acc[i][j][4 * g4 + 1] * sc,
-                                           acc[i][j][4 * g4 + 2] * sc, acc[i][j][4 * g4 + 3] * sc);
-                    if (rr) {
-                        const float4 a = *reinterpret_cast<const float4 *>(rr + m);
-                        v = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
-                    }
-                    *reinterpret_cast<float4 *>(yr + m) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (m + e < M) {
-                            const float v = acc[i][j][4 * g4 + e] * sc;
-                            yr[m + e] = rr ? rr[m + e] + v : v;
-                        }
-                }
-            }
-        }
-}
-
-// gemm_f16_kernel's 256-token tiles in the producer/consumer form of the
-// K loop (k_loop_pc): the same grid, the same tile order and bit-identical
-// results; waves 4-7 hold the sums and write them. (The fused gate/up keeps
-// the 8-wave k_loop: its SiLU epilogue on four waves instead of eight made
-// the 1.8B prefill 2.4 % slower.)
-template <int F>
-__global__ __launch_bounds__(PC_THREADS, 1) void gemm_f16_pc_kernel(
-    GemmSegs g, int K, const _Float16 *__restrict__ xh, const float *__restrict__ rscale, int N,
-    int mtiles, int ntiles, int kslices, float *__restrict__ part)
-{
-    __shared__ __attribute__((aligned(16))) _Float16 lds[lds_halves<8>()];
-    const int T = xcd_tile(mtiles * ntiles);
-    if (T >= mtiles * ntiles) return;
-    int mt = T / ntiles, sg = 0;
-    while (sg + 1 < g.nseg && mt >= g.s[sg].tiles) mt -= g.s[sg++].tiles;
-    const GemmSeg &S = g.s[sg];
-    const int M = S.rows;
-    const int m0 = mt * BM, n0 = (T % ntiles) * 256;
-
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    auto wsrc = [&](int lrow, WView &v, int &row) {
-        v = S.w;
-        row = m0 + lrow < M ? m0 + lrow : -1;
-    };
-    auto xrow = [&](int r) -> const _Float16 * {
-        return n0 + r < N ? xh + (size_t)(n0 + r) * K : nullptr;
-    };
-    const int c = (threadIdx.x >> 6) & 3, wm = c >> 1, wn = c & 1;
-    auto arow = [&](int i) { return wm * 64 + 32 * i; };
-    const int kslice = K / kslices;
-    k_loop_pc<F>(wsrc, xrow, arow, kslice, lds, acc, blockIdx.y * kslice);
-    if (threadIdx.x < 256) return; // the producers
-
-    float *y = kslices > 1 ? part + (size_t)blockIdx.y * N * M : S.y;
-    const float *residual = kslices > 1 ? nullptr : S.residual;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + wn * 128 + 32 * j + (threadIdx.x & 31);
-            if (n >= N) continue;
-            float *yr = y + (size_t)n * M;
-            const float *rr = residual ? residual + (size_t)n * M : nullptr;
-            const float sc = rscale[n];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int m = m0 + wm * 64 + 32 * i + acc_row_in_block(4 * g4);
-                if (m + 3 < M && (M & 3) == 0) {
-                    float4 v = make_float4(acc[i][j][4 * g4] * sc, acc[i][j][4 * g4 + 1] * sc,
-                                           acc[i][j][4 * g4 + 2] * sc, acc[i][j][4 * g4 + 3] * sc);
-                    if (rr) {
-                        const float4 a = *reinterpret_cast<const float4 *>(rr + m);
-                        v = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
-                    }
-                    *reinterpret_cast<float4 *>(yr + m) = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (m + e < M) {
-                            const float v = acc[i][j][4 * g4 + e] * sc;
-                            yr[m + e] = rr ? rr[m + e] + v : v;
-                        }
-                }
-            }
-        }
-}
-
-// The 256-token tiles with the activations, in fragment order
-// (launch_to_f16 with frag), straight into the consumers' registers
-// (k_loop_pcx): the tile order of gemm_f16_pc_kernel over tiles of 32 NI
-// weight rows (128, or 96 where that fills more of the CUs), bit-identical
-// results; consumer wave 4 + c writes tokens 64 c ...
-template <int F, int NI>
-__global__ __launch_bounds__(PC_THREADS, 1) void gemm_f16_pcx_kernel(
-    GemmSegs g, int K, const _Float16 *__restrict__ xh, const float *__restrict__ rscale, int N,
-    int mtiles, int ntiles, int kslices, float *__restrict__ part)
-{
-    __shared__ __attribute__((aligned(16))) _Float16 lds[2 * TILE_HALVES];
-    const int T = xcd_tile(mtiles * ntiles);
-    if (T >= mtiles * ntiles) return;
-    int mt = T / ntiles, sg = 0;
-    while (sg + 1 < g.nseg && mt >= g.s[sg].tiles) mt -= g.s[sg++].tiles;
-    const GemmSeg &S = g.s[sg];
-    const int M = S.rows;
-    const int m0 = mt * (32 * NI), n0 = (T % ntiles) * 256;
-
-    f32x16 acc[NI][2];
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    auto wsrc = [&](int lrow, WView &v, int &row) {
-        v = S.w;
-        row = m0 + lrow < M ? m0 + lrow : -1;
-    };
-    // the fragment-order run of the 32-token block holding tile token r
-    // (clamped into the batch's blocks)
-    auto xsrc = [&](int r) -> const _Float16 * {
-        return xh + (size_t)min((n0 + r) / 32, (N - 1) / 32) * 32 * K;
-    };
-    const int kslice = K / kslices;
-    k_loop_pcx<F, NI>(wsrc, xsrc, kslice, lds, acc, blockIdx.y * kslice);
-    if (threadIdx.x < 256) return; // the producers
-    const int c = (threadIdx.x >> 6) & 3;
-
-    float *y = kslices > 1 ? part + (size_t)blockIdx.y * N * M : S.y;
-    const float *residual = kslices > 1 ? nullptr : S.residual;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + 64 * c + 32 * j + (threadIdx.x & 31);
-            if (n >= N) continue;
-            float *yr = y + (size_t)n * M;
-            const float *rr = residual ? residual + (size_t)n * M : nullptr;
-            const float sc = rscale[n];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int m = m0 + 32 * i + acc_row_in_block(4 * g4);
                 if (m + 3 < M && (M & 3) == 0) {
                     float4 v = make_float4(acc[i][j][4 * g4] * sc, acc[i][j][4 * g4 + 1] * sc,
                                            acc[i][j][4 * g4 + 2] * sc, acc[i][j][4 * g4 + 3] * sc);
@@ -962,108 +860,92 @@ __device__ __forceinline__ float silu_mul(float g, float u)
     return (g / (1.0f + expf(-g))) * u;
 }
 
-// Gate and up of one expert chunk: LDS rows 0..63 dequantize gate rows
-// m0..m0+63 and rows 64..127 the same rows of up; wave (wm, wn) holds gate
-// rows 32*wm.. in acc[0] and the matching up rows in acc[1], so the SiLU
-// product pairs registers one to one. H[q][m] = silu(g) * u in f32, with g
-// and u scaled back by the token row's activation scale.
+// Gate and up of a tile: the first half of the LDS rows (64; 32 for Tile64)
+// dequantizes gate rows m0 .., the second the same rows of up; the first half of a wave's row blocks is
+// gate, the second the matching up rows, so the SiLU product pairs registers
+// one to one. xt: the operand of the tile's first token (cnt of them), with
+// scales xs. h[n][m] = silu(g) * u in f32, g and u scaled back by the token's
+// activation scale (DenseFfn::forward, src/model.rs:679-683); ebase is the
+// first row of an expert's slice of the weights.
+template <int F, class C>
+__device__ __forceinline__ void gate_up_tile(const WView &gate, const WView &up, size_t ebase,
+                                             int mid, int m0, int K, const _Float16 *xt,
+                                             const float *xs, int cnt, float *h, _Float16 *lds)
+{
+    constexpr int HB = C::RB / 2, HR = tile_rows<C>() / 2;
+    const int wr = px_wr<C>();
+    f32x16 acc[C::RB][C::CB];
+    auto wsrc = [&](int lrow, WView &v, int &row) {
+        v = lrow < HR ? gate : up;
+        row = (int)ebase + min(m0 + lrow % HR, mid - 1);
+    };
+    auto arow = [&](int i) { return i < HB ? 32 * (wr * HB + i) : HR + 32 * (wr * HB + i - HB); };
+    if (!k_loop_px<F, C>(wsrc, arow, xt, cnt, K, 0, K, lds, acc)) return;
+#pragma unroll
+    for (int j = 0; j < C::CB; ++j) {
+        const int n = px_token<C>(j);
+        if (n >= cnt) continue;
+        float *hr = h + (size_t)n * mid;
+        const float sc = xs[n];
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                // (mid is a multiple of 4: whole groups of four rows)
+                const int m = m0 + arow(i) + acc_row_in_block(4 * g4);
+                if (m >= mid) continue;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = silu_mul(acc[i][j][4 * g4 + e] * sc, acc[i + HB][j][4 * g4 + e] * sc);
+                *reinterpret_cast<float4 *>(hr + m) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+    }
+}
+
+// An expert's chunk of the MoE pairs against 64 of its gate and up rows.
 template <int F>
-__global__ __launch_bounds__(256, 2) void moe_gate_up_kernel(
+__global__ __launch_bounds__(tile_threads<TileMoe>(), TileMoe::OCC) void moe_gate_up_kernel(
     WView gate, WView up, int mid, int K, const int *__restrict__ eoff,
     const int *__restrict__ tiles, const int *__restrict__ ntiles,
     const _Float16 *__restrict__ xg, const float *__restrict__ xscale, float *__restrict__ H,
     int mtiles, int max_tiles)
 {
-    __shared__ __attribute__((aligned(16))) _Float16 lds[4 * TILE_HALVES];
+    __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
     const int T = xcd_tile(mtiles * max_tiles);
     if (T >= mtiles * max_tiles) return;
     const int ti = T / mtiles, mt = T % mtiles;
     if (ti >= *ntiles) return;
     const int e = tiles[2 * ti], c = tiles[2 * ti + 1];
     const int nb = eoff[e] + c * BN;
-    const int cnt = min(BN, eoff[e + 1] - nb);
-    const int m0 = mt * 64;
-    const int wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
-
-    f32x16 acc[2][2];
-    zero_acc(acc);
-    auto wsrc = [&](int lrow, WView &v, int &row) {
-        const int m = m0 + (lrow & 63);
-        v = lrow < 64 ? gate : up;
-        row = m < mid ? e * mid + m : -1;
-    };
-    auto xrow = [&](int r) -> const _Float16 * {
-        return r < cnt ? xg + (size_t)(nb + r) * K : nullptr;
-    };
-    auto arow = [&](int i) { return 64 * i + 32 * wm; };
-    if (cnt <= 32) k_loop<F, 1>(wsrc, xrow, arow, K, wn, lds, acc);
-    else k_loop<F, 2>(wsrc, xrow, arow, K, wn, lds, acc);
-
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int r = acc_col(wn, j);
-        if (r >= cnt) continue;
-        float *hr = H + (size_t)(nb + r) * mid;
-        const float sc = xscale[nb + r];
-#pragma unroll
-        for (int e4 = 0; e4 < 16; ++e4) {
-            const int m = m0 + 32 * wm + acc_row_in_block(e4);
-            if (m < mid) hr[m] = silu_mul(acc[0][j][e4] * sc, acc[1][j][e4] * sc);
-        }
-    }
+    gate_up_tile<F, TileMoe>(gate, up, (size_t)e * mid, mid, mt * 64, K, xg + (size_t)nb * K,
+                             xscale + nb, min(BN, eoff[e + 1] - nb), H + (size_t)nb * mid, lds);
 }
 
-// Gate and up of a dense FFN at batch N (DenseFfn::forward, src/model.rs:
-// 679-683): the tile pairs gate rows m0..m0+63 with the same rows of up, as
-// moe_gate_up_kernel does, and writes H[n][m] = silu(g) * u in f32 (NW waves,
-// 32 NW tokens per tile, as gemm_f16_kernel).
-template <int F, int NW>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_gate_up_kernel(
+// Gate and up of a dense FFN at batch N.
+template <int F, class C>
+__global__ __launch_bounds__(tile_threads<C>(), C::OCC) void gemm_gate_up_kernel(
     WView gate, WView up, int mid, int K, const _Float16 *__restrict__ xh,
     const float *__restrict__ rscale, int N, float *__restrict__ H, int mtiles, int ntiles)
 {
-    __shared__ __attribute__((aligned(16))) _Float16 lds[lds_halves<NW>()];
+    __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
     const int T = xcd_tile(mtiles * ntiles);
     if (T >= mtiles * ntiles) return;
-    const int m0 = (T / ntiles) * 64, n0 = (T % ntiles) * (32 * NW);
-    const int wave = threadIdx.x >> 6, wm = wave / (NW / 2), wn = wave % (NW / 2);
-
-    f32x16 acc[2][2];
-    zero_acc(acc);
-    auto wsrc = [&](int lrow, WView &v, int &row) {
-        const int m = m0 + (lrow & 63);
-        v = lrow < 64 ? gate : up;
-        row = m < mid ? m : -1;
-    };
-    auto xrow = [&](int r) -> const _Float16 * {
-        return n0 + r < N ? xh + (size_t)(n0 + r) * K : nullptr;
-    };
-    auto arow = [&](int i) { return 64 * i + 32 * wm; };
-    k_loop<F, 2, NW>(wsrc, xrow, arow, K, wn, lds, acc);
-
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = n0 + acc_col(wn, j);
-        if (n >= N) continue;
-        float *hr = H + (size_t)n * mid;
-        const float sc = rscale[n];
-#pragma unroll
-        for (int e4 = 0; e4 < 16; ++e4) {
-            const int m = m0 + 32 * wm + acc_row_in_block(e4);
-            if (m < mid) hr[m] = silu_mul(acc[0][j][e4] * sc, acc[1][j][e4] * sc);
-        }
-    }
+    const int n0 = (T % ntiles) * tile_tokens<C>();
+    gate_up_tile<F, C>(gate, up, 0, mid, (T / ntiles) * (tile_rows<C>() / 2), K, xh + (size_t)n0 * K, rscale + n0,
+                       min(tile_tokens<C>(), N - n0), H + (size_t)n0 * mid, lds);
 }
 
 // Down of one expert chunk: outp[q][m] = down_e[m] . H[q] (H in f16 with its
 // row scale).
 template <int F>
-__global__ __launch_bounds__(256, 2) void moe_down_kernel(
+__global__ __launch_bounds__(tile_threads<TileMoe>(), TileMoe::OCC) void moe_down_kernel(
     WView down, int hidden, int K, const int *__restrict__ eoff, const int *__restrict__ tiles,
     const int *__restrict__ ntiles, const _Float16 *__restrict__ H,
     const float *__restrict__ hscale, float *__restrict__ outp, int mtiles, int max_tiles)
 {
-    __shared__ __attribute__((aligned(16))) _Float16 lds[4 * TILE_HALVES];
+    using C = TileMoe;
+    __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
     const int T = xcd_tile(mtiles * max_tiles);
     if (T >= mtiles * max_tiles) return;
     const int ti = T / mtiles, mt = T % mtiles;
@@ -1072,35 +954,33 @@ __global__ __launch_bounds__(256, 2) void moe_down_kernel(
     const int nb = eoff[e] + c * BN;
     const int cnt = min(BN, eoff[e + 1] - nb);
     const int m0 = mt * BM;
-    const int wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
+    const int wr = px_wr<C>();
 
-    f32x16 acc[2][2];
-    zero_acc(acc);
+    f32x16 acc[C::RB][C::CB];
     auto wsrc = [&](int lrow, WView &v, int &row) {
         v = down;
-        row = m0 + lrow < hidden ? e * hidden + m0 + lrow : -1;
+        row = e * hidden + min(m0 + lrow, hidden - 1);
     };
-    auto xrow = [&](int r) -> const _Float16 * {
-        return r < cnt ? H + (size_t)(nb + r) * K : nullptr;
-    };
-    auto arow = [&](int i) { return wm * 64 + 32 * i; };
-    if (cnt <= 32) k_loop<F, 1>(wsrc, xrow, arow, K, wn, lds, acc);
-    else k_loop<F, 2>(wsrc, xrow, arow, K, wn, lds, acc);
-
+    auto arow = [&](int i) { return 32 * (wr * C::RB + i); };
+    if (!k_loop_px<F, C>(wsrc, arow, H + (size_t)nb * K, cnt, K, 0, K,
+                                                  lds, acc))
+        return;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < C::RB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int r = acc_col(wn, j);
+        for (int j = 0; j < C::CB; ++j) {
+            const int r = px_token<C>(j);
             if (r >= cnt) continue;
             float *orow = outp + (size_t)(nb + r) * hidden;
             const float sc = hscale[nb + r];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                // (hidden is a multiple of 4)
                 const int m = m0 + arow(i) + acc_row_in_block(4 * g);
-#pragma unroll
-                for (int e4 = 0; e4 < 4; ++e4)
-                    if (m + e4 < hidden) orow[m + e4] = acc[i][j][4 * g + e4] * sc;
+                if (m < hidden)
+                    *reinterpret_cast<float4 *>(orow + m) =
+                        make_float4(acc[i][j][4 * g] * sc, acc[i][j][4 * g + 1] * sc,
+                                    acc[i][j][4 * g + 2] * sc, acc[i][j][4 * g + 3] * sc);
             }
         }
 }
@@ -1127,68 +1007,94 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float *__restrict__ ou
 
 } // namespace
 
-int launch_to_f16(const float *x, int rows, int K, _Float16 *xh, float *rscale, void *stream,
-                  bool frag)
+int launch_to_f16(const float *x, int rows, int K, _Float16 *xh, float *rscale, void *stream)
 {
-    if (!frag) return launch_norm_to_f16(x, rows, K, nullptr, 0.f, xh, rscale, stream);
-    if (rows <= 0) return 0;
-    if (K % 16) return (int)hipErrorInvalidValue;
-    launch_rows_to_f16(rows, K, (hipStream_t)stream, x, nullptr, nullptr, nullptr, nullptr, 0.f,
-                       xh, rscale, true);
-    return (int)hipGetLastError();
+    return launch_norm_to_f16(x, rows, K, nullptr, 0.f, xh, rscale, stream);
 }
 
 int launch_norm_to_f16(const float *x, int rows, int K, const float *norm, float eps,
                        _Float16 *xh, float *rscale, void *stream)
 {
     if (rows <= 0) return 0;
-    if (K % 4) return (int)hipErrorInvalidValue;
+    if (K % 16) return (int)hipErrorInvalidValue;
     launch_rows_to_f16(rows, K, (hipStream_t)stream, x, nullptr, nullptr, nullptr, norm, eps, xh,
-                       rscale, false);
+                       rscale);
     return (int)hipGetLastError();
 }
 
-// Waves per dense GEMM workgroup: 8 (256-token tiles, each dequantized
-// weight slice feeding twice the MFMAs) when the batch exceeds one 128-token
-// tile and the 8-wave grid (`tiles` row tiles x K slices, times the 256-token
-// tiles) still gives at least 3/4 of the 256 CUs a workgroup; else 4 (two
-// workgroups per CU). Measured: Q4_K [14336 x 4096] x 512 tokens 120 -> 100
-// us, while grids of 64-96 workgroups ran 6-13 % slower with 8 waves. Both
-// forms give every element the same result, so the choice is free.
-int gemm_waves(int batch, int tiles)
+namespace {
+
+enum TileShape { T256, T256R96, T192, T128, T64 };
+
+// The tile shape of a dense product: the one whose workgroups take the least
+// time in rounds over the 256 CUs. rows(r): row tiles of r rows. A shape's
+// time is that of a 64-column step with one workgroup on a CU (us, Q4_K
+// [14336 x 4096]: 67 us for 64 steps of 224 workgroups of 256 tokens), `pair`
+// with two (Tile128, Tile64). All shapes give an element the same bits, so the
+// choice is free. By 256, 192, 128 tokens and 64 rows x 256 tokens: Q2_0C
+// [12288 x 2048] at 777 tokens 71 / 67 / 71 / 63 us, Q4_K [14336 x 4096] at
+// 130 tokens 57 / 52 / 47 / 40 us, 384: 71 / 66 / 78 / 76, 512: 77 / 109 / 88
+// / 83, 777: 130 / 147 / 142 / 136.
+template <class Rows> TileShape pick_tile(int batch, int kslices, bool r96, const Rows &rows)
 {
-    return batch > BN && (size_t)tiles * ((batch + 255) / 256) >= 192 ? 8 : 4;
+    struct Shape {
+        TileShape s;
+        int rows, tokens;
+        float time, pair;
+    };
+    static constexpr Shape shapes[] = {{T256, 128, 256, 1.06f, 0.f},
+                                       {T256R96, 96, 256, 0.85f, 0.f},
+                                       {T192, 128, 192, 0.9f, 0.f},
+                                       {T128, 128, 128, 0.73f, 1.25f},
+                                       {T64, 64, 256, 0.5f, 1.08f}};
+    TileShape best = T256;
+    float least = 1e30f;
+    for (const Shape &c : shapes) {
+        if (c.s == T256R96 && !r96) continue;
+        const long wgs = (long)rows(c.rows) * ((batch + c.tokens - 1) / c.tokens) * kslices;
+        const long full = c.pair ? wgs / 512 : wgs / 256, rest = c.pair ? wgs % 512 : wgs % 256;
+        const float time = (float)full * (c.pair ? c.pair : c.time) +
+                           (rest == 0 ? 0.f : rest <= 256 ? c.time : c.pair);
+        if (time < least) {
+            least = time;
+            best = c.s;
+        }
+    }
+    return best;
 }
+
+} // namespace
 
 int launch_gate_up_f16(int fmt, WView gate, WView up, int cols, const _Float16 *xh,
                        const float *rscale, int batch, float *h, void *stream)
 {
-    if (cols % BK) return (int)hipErrorInvalidValue;
+    if (cols % BK || gate.rows % 4) return (int)hipErrorInvalidValue;
     const int mid = gate.rows;
-    const int mtiles = (mid + 63) / 64;
-    const int nw = gemm_waves(batch, mtiles), bn = 32 * nw;
-    const int ntiles = (batch + bn - 1) / bn;
-    const int per = (mtiles * ntiles + 7) / 8;
-    dim3 grid(8 * per), block(64 * nw);
+    auto row_tiles = [&](int r) { return (mid + r / 2 - 1) / (r / 2); };
+    const TileShape shape = pick_tile(batch, 1, false, row_tiles);
     hipStream_t st = (hipStream_t)stream;
-#define HYQ_GU(F)                                                                              \
-    case F:                                                                                    \
-        if (nw == 8)                                                                           \
-            hipLaunchKernelGGL((gemm_gate_up_kernel<F, 8>), grid, block, 0, st, gate, up, mid,  \
-                               cols, xh, rscale, batch, h, mtiles, ntiles);                    \
-        else                                                                                   \
-            hipLaunchKernelGGL((gemm_gate_up_kernel<F, 4>), grid, block, 0, st, gate, up, mid,  \
-                               cols, xh, rscale, batch, h, mtiles, ntiles);                    \
-        break;
+    auto launch = [&](auto fc, auto cc) {
+        using C = decltype(cc);
+        const int mtiles = row_tiles(tile_rows<C>());
+        const int ntiles = (batch + tile_tokens<C>() - 1) / tile_tokens<C>();
+        const dim3 grid((mtiles * ntiles + 7) / 8 * 8);
+        hipLaunchKernelGGL((gemm_gate_up_kernel<fc(), C>), grid, dim3(tile_threads<C>()), 0, st, gate,
+                           up, mid, cols, xh, rscale, batch, h, mtiles, ntiles);
+    };
+    auto run = [&](auto fc) {
+        if (shape == T256) launch(fc, Tile256{});
+        else if (shape == T192) launch(fc, Tile192{});
+        else if (shape == T64) launch(fc, Tile64{});
+        else launch(fc, Tile128{});
+    };
     switch (fmt) {
-        HYQ_GU(Q4_K)
-        HYQ_GU(Q6_K)
-        HYQ_GU(Q8_0)
-        HYQ_GU(Q2_0C)
-        HYQ_GU(STQ1_0)
+    case Q4_K: run(std::integral_constant<int, Q4_K>{}); break;
+    case Q6_K: run(std::integral_constant<int, Q6_K>{}); break;
+    case Q8_0: run(std::integral_constant<int, Q8_0>{}); break;
+    case Q2_0C: run(std::integral_constant<int, Q2_0C>{}); break;
+    case STQ1_0: run(std::integral_constant<int, STQ1_0>{}); break;
     default: return (int)hipErrorInvalidValue;
     }
-#undef HYQ_GU
     return (int)hipGetLastError();
 }
 
@@ -1236,14 +1142,6 @@ int matmul_kslices(int fmt, int M, int K, int batch)
     return base;
 }
 
-bool gemm_frag_operand(int fmt, int rows, int cols, int batch, int kslices)
-{
-    (void)fmt;
-    (void)cols;
-    const int mtiles = (rows + BM - 1) / BM;
-    return gemm_waves(batch, mtiles * (kslices > 1 ? kslices : 1)) == 8;
-}
-
 int launch_gemm_reduce(const float *part, int kslices, size_t count, const float *residual,
                        float *y, void *stream)
 {
@@ -1257,7 +1155,7 @@ int launch_gemm_reduce(const float *part, int kslices, size_t count, const float
 
 int launch_gemm_f16(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale,
                     int batch, float *y, const float *residual, void *stream, float *part,
-                    size_t part_floats, int kslices, bool xfrag)
+                    size_t part_floats, int kslices)
 {
     GemmSegs g{};
     g.nseg = 1;
@@ -1267,69 +1165,53 @@ int launch_gemm_f16(int fmt, WView w, int cols, const _Float16 *xh, const float 
     g.s[0].rows = w.rows;
     const int ks = kslices > 0 ? kslices : gemm_kslices(fmt, w.rows, cols);
     if (ks > 1 && part && part_floats >= (size_t)ks * batch * w.rows) {
-        int rc = launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, ks, part, xfrag);
+        int rc = launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, ks, part);
         if (rc) return rc;
         return launch_gemm_reduce(part, ks, (size_t)batch * w.rows, residual, y, stream);
     }
-    return launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, 1, nullptr, xfrag);
+    return launch_gemm_f16_segs(fmt, g, cols, xh, rscale, batch, stream, 1, nullptr);
 }
 
 int launch_gemm_f16_segs(int fmt, GemmSegs g, int cols, const _Float16 *xh, const float *rscale,
-                         int batch, void *stream, int kslices, float *part, bool xfrag)
+                         int batch, void *stream, int kslices, float *part)
 {
     if (cols % BK || g.nseg < 1 || g.nseg > 3) return (int)hipErrorInvalidValue;
     if (kslices < 1 || (kslices > 1 && (g.nseg != 1 || !part || cols % kslices)))
         return (int)hipErrorInvalidValue;
-    int mtiles = 0;
-    for (int i = 0; i < g.nseg; ++i) {
-        if (i + 1 < g.nseg && g.s[i].rows % BM) return (int)hipErrorInvalidValue;
-        g.s[i].tiles = (g.s[i].rows + BM - 1) / BM;
-        mtiles += g.s[i].tiles;
-    }
-    const int nw = gemm_waves(batch, mtiles * kslices), bn = 32 * nw;
-    // fragment-order activations: only the 256-token tiles of one weight
-    if (xfrag && (nw != 8 || g.nseg != 1 || cols % 16)) return (int)hipErrorInvalidValue;
-    const int ntiles = (batch + bn - 1) / bn;
-    // The fragment-order kernel takes 96-row tiles where they need fewer
-    // rounds of workgroups over the 256 CUs per row of a tile (rounds x tile
-    // rows): a [6144 x 4096] product in two K slices at 512 tokens runs as
-    // 64 x 2 x 2 = 256 workgroups of 96 rows instead of 192 of 128.
-    bool rows96 = false;
-    if (xfrag) {
-        const int m96 = (g.s[0].rows + 95) / 96;
-        auto rounds = [&](int mt) { return (mt * ntiles * kslices + 255) / 256; };
-        if (rounds(m96) * 96 < rounds(mtiles) * BM) {
-            rows96 = true;
-            mtiles = g.s[0].tiles = m96;
-        }
-    }
-    const int per = (mtiles * ntiles + 7) / 8;
-    dim3 grid(8 * per, kslices), block(64 * nw);
+    for (int i = 0; i + 1 < g.nseg; ++i)
+        if (g.s[i].rows % BM) return (int)hipErrorInvalidValue;
+    auto row_tiles = [&](int r) {
+        int mt = 0;
+        for (int i = 0; i < g.nseg; ++i) mt += (g.s[i].rows + r - 1) / r;
+        return mt;
+    };
+    const TileShape shape = pick_tile(batch, kslices, g.nseg == 1, row_tiles);
     hipStream_t st = (hipStream_t)stream;
-#define HYQ_GEMM(F)                                                                            \
-    case F:                                                                                    \
-        if (xfrag && rows96)                                                                   \
-            hipLaunchKernelGGL((gemm_f16_pcx_kernel<F, 3>), grid, block, 0, st, g, cols, xh,    \
-                               rscale, batch, mtiles, ntiles, kslices, part);                  \
-        else if (xfrag)                                                                        \
-            hipLaunchKernelGGL((gemm_f16_pcx_kernel<F, 4>), grid, block, 0, st, g, cols, xh,    \
-                               rscale, batch, mtiles, ntiles, kslices, part);                  \
-        else if (nw == 8)                                                                      \
-            hipLaunchKernelGGL((gemm_f16_pc_kernel<F>), grid, block, 0, st, g, cols, xh,        \
-                               rscale, batch, mtiles, ntiles, kslices, part);                  \
-        else                                                                                   \
-            hipLaunchKernelGGL((gemm_f16_kernel<F, 4>), grid, block, 0, st, g, cols, xh, rscale, \
-                               batch, mtiles, ntiles, kslices, part);                          \
-        break;
+    auto launch = [&](auto fc, auto cc) {
+        using C = decltype(cc);
+        for (int i = 0; i < g.nseg; ++i)
+            g.s[i].tiles = (g.s[i].rows + tile_rows<C>() - 1) / tile_rows<C>();
+        const int mtiles = row_tiles(tile_rows<C>());
+        const int ntiles = (batch + tile_tokens<C>() - 1) / tile_tokens<C>();
+        const dim3 grid((mtiles * ntiles + 7) / 8 * 8, kslices);
+        hipLaunchKernelGGL((gemm_f16_kernel<fc(), C>), grid, dim3(tile_threads<C>()), 0, st, g, cols, xh,
+                           rscale, batch, mtiles, ntiles, kslices, part);
+    };
+    auto run = [&](auto fc) {
+        if (shape == T256) launch(fc, Tile256{});
+        else if (shape == T256R96) launch(fc, Tile256R96{});
+        else if (shape == T192) launch(fc, Tile192{});
+        else if (shape == T64) launch(fc, Tile64{});
+        else launch(fc, Tile128{});
+    };
     switch (fmt) {
-        HYQ_GEMM(Q4_K)
-        HYQ_GEMM(Q6_K)
-        HYQ_GEMM(Q8_0)
-        HYQ_GEMM(Q2_0C)
-        HYQ_GEMM(STQ1_0)
+    case Q4_K: run(std::integral_constant<int, Q4_K>{}); break;
+    case Q6_K: run(std::integral_constant<int, Q6_K>{}); break;
+    case Q8_0: run(std::integral_constant<int, Q8_0>{}); break;
+    case Q2_0C: run(std::integral_constant<int, Q2_0C>{}); break;
+    case STQ1_0: run(std::integral_constant<int, STQ1_0>{}); break;
     default: return (int)hipErrorInvalidValue;
     }
-#undef HYQ_GEMM
     return (int)hipGetLastError();
 }
 
@@ -1459,11 +1341,11 @@ int launch_moe(int fmt_gu, int fmt_down, WView gate, WView up, WView down, int h
         return (int)hipGetLastError();
     }
     launch_rows_to_f16(npairs, hidden, st, x, order, ptok, eoff + experts, nullptr, 0.f, xg,
-                       xscale, false);
+                       xscale, pexp, eoff);
     {
         const int mtiles = (mid + 63) / 64;
         const int per = (mtiles * L.max_tiles + 7) / 8;
-        dim3 grid(8 * per), block(256);
+        dim3 grid(8 * per), block(tile_threads<TileMoe>());
 #define HYQ_MOE_GU(F)                                                                          \
     case F:                                                                                    \
         hipLaunchKernelGGL(moe_gate_up_kernel<F>, grid, block, 0, st, gate, up, mid, hidden,   \
@@ -1479,12 +1361,12 @@ int launch_moe(int fmt_gu, int fmt_down, WView gate, WView up, WView down, int h
         }
 #undef HYQ_MOE_GU
     }
-    launch_rows_to_f16(npairs, mid, st, h32, nullptr, nullptr, eoff + experts, nullptr, 0.f, H,
-                       hscale, false);
+    launch_rows_to_f16(npairs, mid, st, h32, order, nullptr, eoff + experts, nullptr, 0.f, H,
+                       hscale, pexp, eoff);
     {
         const int mtiles = (hidden + BM - 1) / BM;
         const int per = (mtiles * L.max_tiles + 7) / 8;
-        dim3 grid(8 * per), block(256);
+        dim3 grid(8 * per), block(tile_threads<TileMoe>());
 #define HYQ_MOE_DN(F)                                                                          \
     case F:                                                                                    \
         hipLaunchKernelGGL(moe_down_kernel<F>, grid, block, 0, st, down, hidden, mid, eoff,     \

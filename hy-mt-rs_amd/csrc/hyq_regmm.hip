@@ -13,16 +13,19 @@ extern template int launch_regmm_format<Q6_K>(const regmm::Args &, int, void *);
 extern template int launch_regmm_format<Q8_0>(const regmm::Args &, int, void *);
 
 // Up to one or two 32-token blocks, so one workgroup per row tile: past them
-// the weights are dequantized again per 64 tokens and the LDS engine is as
-// fast (Q4_K [14336 x 4096] at 128 tokens 47.7 against 52 us, Q2_0C
-// [2048 x 6144] 33 against 32). Q6_K's second block does not fit the
-// registers (spilled, [4096 x 14336] at 64 tokens 66 against 51 us). At least
-// four 64-column steps per wave: a narrower weight leaves the waves that
-// split its columns without work to overlap.
+// the weights are dequantized again per 64 tokens and the LDS engine is
+// faster (Q4_K [14336 x 4096] at 128 tokens 47.7 against 38 us). Q6_K's second
+// block does not fit the registers (spilled, [4096 x 14336] at 64 tokens 66
+// against 40 us), and its widest weights, whose row tiles leave a CU one
+// workgroup of four waves, are faster in the engine's producers ([4096 x
+// 14336] at 30 tokens 36.5 against 28.7 us; [14336 x 4096] 25.3 against 26.7,
+// [2048 x 2048] 13.5 against 14.5). At least four 64-column steps per wave: a
+// narrower weight leaves the waves that split its columns without work to
+// overlap.
 bool regmm_fits(int fmt, int cols, int batch)
 {
     return batch >= 2 && batch <= (fmt == Q6_K ? 32 : 64) && cols % tile::BK == 0 &&
-           cols / tile::BK >= 4 * regmm::WAVES;
+           cols / tile::BK >= 4 * regmm::WAVES && (fmt != Q6_K || cols < 8192);
 }
 
 // K slices across workgroups, where the row tiles leave CUs without one: to

@@ -25,8 +25,8 @@
 // a 16-deep step may take its columns in any order as long as both operands
 // take the same - so the token fragments, kept in fragment order (8
 // consecutive columns of a token per 16-byte piece), are read at the pieces
-// of those columns. The packed bytes of the next D steps are in registers
-// while one is multiplied.
+// of those columns. The packed bytes of the next 256 columns are in registers
+// while 256 are multiplied.
 //
 // Every weight is the same f16 value as in the LDS engine (one fma
 // bit-identical to the decoder, one rounding); an output's terms are summed
@@ -46,22 +46,24 @@ namespace regmm {
 using namespace tile;
 
 // The 8-column piece (of the 64-column step's eight) that fragment i of half
-// h holds, as an offset in halves into the step's fragment-order run: piece g
-// is at (g / 2) * 512 + (g % 2) * 256.
+// h holds: piece g of a block of c tokens is at 8 c g halves of the step's
+// fragment-order run.
 template <int F> __device__ constexpr int piece(int i, int h)
 {
-    const int c = i < 2 ? Deq<F>::c0(h) + 8 * i : Deq<F>::c1(h) + 8 * (i - 2);
-    return (c / 16) * 512 + (c / 8 % 2) * 256;
+    return (i < 2 ? Deq<F>::c0(h) + 8 * i : Deq<F>::c1(h) + 8 * (i - 2)) / 8;
 }
-
-// Steps of packed bytes in flight per wave: as many as the registers hold.
-template <int F, int TB> constexpr int depth() { return F == Q6_K || TB > 1 ? 2 : 4; }
 
 // Waves of a workgroup. Four, so that a CU holds up to four workgroups at the
 // 128 registers of a wave and one's loads run under another's products; with
 // 8 and 16 waves Q4_K [14336 x 4096] at 21 tokens took 24.9 and 28.7 us
 // against 23.4.
 constexpr int WAVES = 4;
+
+// Waves per SIMD: what two 256-column blocks of packed bytes leave room for.
+template <int F, int TB> constexpr int occupancy()
+{
+    return F == Q6_K || (TB > 1 && (F == Q4_K || F == Q8_0)) ? 3 : 4;
+}
 
 struct Args {
     GemmSegs g; // .tiles: row tiles of 32 rows
@@ -72,10 +74,9 @@ struct Args {
 };
 
 template <int F, int TB>
-__global__ __launch_bounds__(64 * WAVES, 4) void regmm_kernel(Args a)
+__global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel(Args a)
 {
     using D = Deq<F>;
-    constexpr int DEPTH = depth<F, TB>();
     __shared__ float4 red[TB][WAVES][4][64];
     const int total = a.rtiles * a.groups, per = (total + 7) / 8;
     const int T = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8); // XCD-contiguous
@@ -89,10 +90,12 @@ __global__ __launch_bounds__(64 * WAVES, 4) void regmm_kernel(Args a)
     const int t = threadIdx.x, lane = t & 63, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
-    // this wave's steps
-    const int steps = K / BK, z = blockIdx.y;
-    const int z0 = (int)((long)steps * z / a.kslices), z1 = (int)((long)steps * (z + 1) / a.kslices);
-    const int c0 = z0 + (z1 - z0) * wave / WAVES, c1 = z0 + (z1 - z0) * (wave + 1) / WAVES;
+    // this wave's steps, whole 256-column blocks of four (Q8_0's last may be less)
+    const int steps = K / BK, blocks = (steps + 3) / 4, z = blockIdx.y;
+    const int z0 = (int)((long)blocks * z / a.kslices);
+    const int z1 = (int)((long)blocks * (z + 1) / a.kslices);
+    const int b0 = z0 + (z1 - z0) * wave / WAVES, b1 = z0 + (z1 - z0) * (wave + 1) / WAVES;
+    const int c0 = 4 * b0, c1 = min(4 * b1, steps);
 
     f32x16 acc[TB];
 #pragma unroll
@@ -106,31 +109,34 @@ __global__ __launch_bounds__(64 * WAVES, 4) void regmm_kernel(Args a)
         const int nblk = (N + 31) / 32;
         // piece(i, h) = piece(i, 0) + h * (piece(0, 1) - piece(0, 0))
         const int hoff = h * (piece<F>(0, 1) - piece<F>(0, 0));
+        unsigned pstride[TB]; // halves per piece of the block
 #pragma unroll
-        for (int b = 0; b < TB; ++b)
-            xb[b] = a.xh + (size_t)min(n0 / 32 + b, nblk - 1) * 32 * K + (lane & 31) * 8 + hoff;
-        typename D::Raw raw[DEPTH];
+        for (int b = 0; b < TB; ++b) {
+            const int blk = min(n0 / 32 + b, nblk - 1), c = min(32, N - 32 * blk);
+            pstride[b] = 8 * c;
+            xb[b] = a.xh + (size_t)blk * 32 * K + min(lane & 31, c - 1) * 8 + hoff * 8 * c;
+        }
+        typename D::Raw raw[2];
         half8 B[2][TB][2]; // fragments 0, 1 and 2, 3 of a step
+        auto load_w = [&](int i, int b) { D::load(raw[i], rp, 4 * min(b, b1 - 1), c1 - 1, h); };
         auto load_b = [&](int s, int c) {
 #pragma unroll
             for (int b = 0; b < TB; ++b)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    B[s][b][i] = *reinterpret_cast<const half8 *>(xb[b] + (size_t)c * 2048 +
-                                                                  piece<F>(2 * s + i, 0));
+                    B[s][b][i] = *reinterpret_cast<const half8 *>(
+                        xb[b] + (8u * c + piece<F>(2 * s + i, 0)) * pstride[b]);
         };
+        // (straight-line blocks left only at the loop's end: see px_produce)
+        auto block = [&](int d, int b, int n) {
+            load_w(d ^ 1, b + 1);
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) D::load(raw[d], rp, min(c0 + d, c1 - 1) * BK, h);
-        load_b(0, c0);
-        for (int cb = c0; cb < c1; cb += DEPTH) {
-#pragma unroll
-            for (int d = 0; d < DEPTH; ++d) {
-                const int c = cb + d;
-                if (c >= c1) break;
+            for (int u = 0; u < 4; ++u) {
+                if (F == Q8_0 && u >= n) return;
+                const int c = 4 * b + u;
                 load_b(1, c);
                 half8 w[4];
-                D::values(raw[d], c & 3, h, w);
-                D::load(raw[d], rp, min(c + DEPTH, c1 - 1) * BK, h);
+                D::values(raw[d], u, h, w);
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -142,6 +148,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void regmm_kernel(Args a)
                     if (s == 0) load_b(0, min(c + 1, c1 - 1));
                 }
             }
+        };
+        load_w(0, b0);
+        load_b(0, c0);
+        for (int b = b0;; b += 2) {
+            block(0, b, c1 - 4 * b);
+            if (b + 1 >= b1) break;
+            block(1, b + 1, c1 - 4 * (b + 1));
+            if (b + 2 >= b1) break;
         }
     }
 

@@ -2,24 +2,14 @@
 // Weight::matmul batch >= 2, src/quant.rs:272-344, and the MoE expert
 // products, src/model.rs:699-725).
 //
-// A workgroup of 256 threads (4 waves) owns BM = 128 LDS weight rows by
-// BN = 128 tokens and walks K in BK = 64 steps:
-//   1. every thread fetches the packed bytes of 32 weights of one LDS row
-//      (row t/2, half t%2) of the next 64-column slice, and 4 x 16 bytes of
-//      the f16 activation slice, into registers (Raw / XRaw);
-//   2. after the current slice's MFMAs it dequantizes them into the other
-//      LDS buffer with the reference decoder's f32 arithmetic
-//      (decode_unchecked, src/quant.rs:2405-2486) and one f32->f16 rounding;
-//   3. each wave multiplies a 64 x 64 (weight rows x tokens) sub-tile with
-//      2 x 2 v_mfma_f32_32x32x16_f16 blocks per 16-wide k step, in f32.
-// Two LDS buffers let one barrier per step separate writers from readers.
+// A workgroup owns up to BM = 128 weight rows by up to 256 tokens and walks K
+// in BK = 64 steps: producer waves fetch the packed bytes of the next steps
+// and dequantize a step's 64 columns into one of two LDS buffers with the
+// reference decoder's f32 arithmetic (decode_unchecked, src/quant.rs:
+// 2405-2486) and one f32->f16 rounding, while consumer waves multiply the
+// other with v_mfma_f32_32x32x16_f16, in f32 (k_loop_px).
 // LDS rows are padded to 72 halves (144 bytes), so the 16-byte fragment
 // reads of 8 consecutive rows fall on 8 distinct 4-bank windows.
-// The wide form (NW = 8 waves, 512 threads) takes 256 tokens: waves 0-3
-// dequantize the weight slice as above, all eight fetch the activations and
-// each multiplies its own 64 x 64 sub-tile, so a dequantized weight feeds
-// twice the MFMAs. Every output element sees the same operands in the same
-// k order in both forms, so their results are bit-identical.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -34,6 +24,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 128, BK = 64, LDK = BK + 8;
 constexpr int TILE_HALVES = BM * LDK; // one LDS operand buffer (BM == BN)
@@ -49,12 +40,17 @@ __device__ __forceinline__ float h2f(uint32_t bits16)
 __device__ __forceinline__ uint32_t byte_of(uint32_t dw, int i) { return (dw >> (8 * i)) & 0xffu; }
 
 // ---------------------------------------------------------------------------
-// Per-format dequantization of 32 weights of one row, columns [k0, k0 + 64)
-// half h: w[0], w[1] hold the columns c0(h) .. c0(h) + 15 of the slice and
-// w[2], w[3] the columns c1(h) .. c1(h) + 15 (which 32 a half takes depends
-// on the format; the two halves of a row cover all 64). load() only issues
-// global loads from the row's plane bases (RowPtr, computed once per thread);
-// values() does the arithmetic from registers, u = (k0 / 64) % 4.
+// Per-format dequantization of a row's weights by two lanes, 32 of every 64
+// columns (a step) each: half h holds the columns c0(h) .. c0(h) + 15 and
+// c1(h) .. c1(h) + 15 of a step (which 32 a half takes depends on the format;
+// the two halves of a row cover all 64). load() only issues global loads from
+// the row's plane bases (RowPtr, computed once per thread), for the four steps
+// s .. s + 3 at once: a row's bytes of 256 columns are one 128-byte line or
+// two, which a load per step would fetch from L2 again at each (Q4_K
+// [14336 x 4096] at 512 tokens moved 66 KB per step and CU so, of which 37
+// were its own). s is a multiple of 4 but for Q8_0, whose rows may end within
+// the four: their steps past `last` read it again. values() does the
+// arithmetic from registers, for step u of the four.
 //
 // Every value is formed as one fma whose exact result is the decoder's
 // exact value, so the f32 result is bit-identical to decode_unchecked
@@ -80,6 +76,9 @@ __device__ __forceinline__ float ub(uint32_t x, int i) { return (float)((x >> (8
 // Eight codes (the bytes of lo, then of hi) as f16(d * q + o).
 __device__ __forceinline__ half8 deq8(uint32_t lo, uint32_t hi, float d, float o)
 {
+    // (the dwords as they are: else each byte is first extracted on its own,
+    // instead of by its v_cvt_f32_ubyteN)
+    asm("" : "+v"(lo), "+v"(hi));
     half8 r;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -96,8 +95,9 @@ __device__ __forceinline__ half8 deq8(uint32_t lo, uint32_t hi, float d, float o
 
 template <int F> struct Deq;
 
-// The values rounded to f16 at their columns of dst (an LDS row).
-template <int F>
+// The values rounded to f16 at their columns of dst (an LDS row): the half's
+// columns c0 .. (PART 0), c1 .. (PART 1) or both (PART -1).
+template <int F, int PART>
 __device__ __forceinline__ void convert(const typename Deq<F>::Raw &r, int u, int h,
                                         _Float16 *dst)
 {
@@ -105,10 +105,14 @@ __device__ __forceinline__ void convert(const typename Deq<F>::Raw &r, int u, in
     Deq<F>::values(r, u, h, w);
     half8 *p0 = reinterpret_cast<half8 *>(dst + Deq<F>::c0(h));
     half8 *p1 = reinterpret_cast<half8 *>(dst + Deq<F>::c1(h));
-    p0[0] = w[0];
-    p0[1] = w[1];
-    p1[0] = w[2];
-    p1[1] = w[3];
+    if constexpr (PART != 1) {
+        p0[0] = w[0];
+        p0[1] = w[1];
+    }
+    if constexpr (PART != 0) {
+        p1[0] = w[2];
+        p1[1] = w[3];
+    }
 }
 
 // Q4_K (decode_unchecked, src/quant.rs:2437-2461): byte l of a 64-weight
@@ -117,7 +121,7 @@ __device__ __forceinline__ void convert(const typename Deq<F>::Raw &r, int u, in
 // 16h..16h+15, i.e. columns 16h.. and 32+16h...
 template <> struct Deq<Q4_K> {
     struct Raw {
-        uint4 q, meta;
+        u32x4 q[4], meta;
     };
     __device__ static constexpr int c0(int h) { return 16 * h; }
     __device__ static constexpr int c1(int h) { return 32 + 16 * h; }
@@ -125,13 +129,15 @@ template <> struct Deq<Q4_K> {
     {
         return row_ptr(w, 128, 16, 0, row);
     }
-    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int k0, int h)
+    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int s, int, int h)
     {
-        const int blk = k0 >> 8, c = (k0 >> 6) & 3;
-        r.q = *reinterpret_cast<const uint4 *>(p.p0 + blk * 128 + 32 * c + 16 * h);
-        r.meta = *reinterpret_cast<const uint4 *>(p.p1 + blk * 16);
+        const int blk = s >> 2;
+        r.meta = *reinterpret_cast<const u32x4 *>(p.p1 + blk * 16);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            r.q[c] = *reinterpret_cast<const u32x4 *>(p.p0 + blk * 128 + 32 * c + 16 * h);
     }
-    __device__ __forceinline__ static void scale_min(const uint4 &meta, int j, int &s, int &m)
+    __device__ __forceinline__ static void scale_min(const u32x4 &meta, int j, int &s, int &m)
     {
         auto sc = [&](int i) -> int {
             const uint32_t dw = i < 4 ? meta.y : i < 8 ? meta.z : meta.w;
@@ -154,7 +160,7 @@ template <> struct Deq<Q4_K> {
         scale_min(r.meta, 2 * c + 1, s1, m1);
         const float da = d * (float)s0, nm1a = -(dmin * (float)m0);
         const float db = d * (float)s1, nm1b = -(dmin * (float)m1);
-        const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
+        const uint32_t q[4] = {r.q[u].x, r.q[u].y, r.q[u].z, r.q[u].w};
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const uint32_t x = q[2 * i], y = q[2 * i + 1];
@@ -170,8 +176,8 @@ template <> struct Deq<Q4_K> {
 // holds planes p0, p0+1 (p0 even); half h takes plane p0 + h.
 template <> struct Deq<Q6_K> {
     struct Raw {
-        uint4 l0, l1, g0, g1;
-        uint32_t sc, d;
+        u32x4 l[2][2], g[2][2], sc; // by 128-weight chunk
+        uint32_t d;
     };
     __device__ static constexpr int c0(int h) { return 32 * h; }
     __device__ static constexpr int c1(int h) { return 32 * h + 16; }
@@ -179,27 +185,34 @@ template <> struct Deq<Q6_K> {
     {
         return row_ptr(w, 192, 16, 2, row);
     }
-    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int k0, int h)
+    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int s, int, int h)
     {
-        const int blk = k0 >> 8, kb = k0 & 255, chunk = kb >> 7;
-        const int pl = 2 * ((kb >> 6) & 1) + h;
+        const int blk = s >> 2;
         const uint8_t *base = p.p0 + blk * 192;
-        r.l0 = *reinterpret_cast<const uint4 *>(base + chunk * 64 + 32 * h);
-        r.l1 = *reinterpret_cast<const uint4 *>(base + chunk * 64 + 32 * h + 16);
-        r.g0 = *reinterpret_cast<const uint4 *>(base + 128 + chunk * 32);
-        r.g1 = *reinterpret_cast<const uint4 *>(base + 128 + chunk * 32 + 16);
-        r.sc = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 16 + chunk * 8 + 2 * pl);
+        r.sc = *reinterpret_cast<const u32x4 *>(p.p1 + blk * 16);
         r.d = *reinterpret_cast<const uint16_t *>(p.p2 + blk * 2);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                r.l[c][i] = *reinterpret_cast<const u32x4 *>(base + c * 64 + 32 * h + 16 * i);
+                r.g[c][i] = *reinterpret_cast<const u32x4 *>(base + 128 + c * 32 + 16 * i);
+            }
     }
     __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
-        const int pl = 2 * (u & 1) + h;
+        const int chunk = u >> 1, pl = 2 * (u & 1) + h;
         const float d = h2f(r.d);
-        const float s0 = d * (float)(int8_t)(r.sc & 0xff), s1 = d * (float)(int8_t)(r.sc >> 8);
+        // scales 2 pl and 2 pl + 1 of the chunk's eight
+        const uint32_t sc = r.sc[2 * chunk + (u & 1)] >> (16 * h);
+        const float s0 = d * (float)(int8_t)(sc & 0xff), s1 = d * (float)(int8_t)(sc >> 8);
         const float o0 = -32.f * s0, o1 = -32.f * s1;
-        const uint32_t ql[8] = {r.l0.x, r.l0.y, r.l0.z, r.l0.w, r.l1.x, r.l1.y, r.l1.z, r.l1.w};
-        const uint32_t qh[8] = {r.g0.x, r.g0.y, r.g0.z, r.g0.w, r.g1.x, r.g1.y, r.g1.z, r.g1.w};
-        const int lsh = (pl >> 1) * 4, hsh = 2 * pl;
+        const u32x4 &l0 = r.l[chunk][0], &l1 = r.l[chunk][1], &g0 = r.g[chunk][0],
+                    &g1 = r.g[chunk][1];
+        const uint32_t ql[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
+        const uint32_t qh[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+        // (pl >> 1 is the step's parity)
+        const int lsh = (u & 1) * 4, hsh = 2 * pl;
         auto codes = [&](int i) {
             return ((ql[i] >> lsh) & 0x0F0F0F0Fu) | (((qh[i] >> hsh) & 0x03030303u) << 4);
         };
@@ -214,8 +227,8 @@ template <> struct Deq<Q6_K> {
 // Q8_0 (src/quant.rs:2409-2414): value = d * q; half h takes the 32-block h.
 template <> struct Deq<Q8_0> {
     struct Raw {
-        uint4 a, b;
-        uint32_t d;
+        u32x4 a[4], b[4];
+        uint32_t d[4];
     };
     __device__ static constexpr int c0(int h) { return 32 * h; }
     __device__ static constexpr int c1(int h) { return 32 * h + 16; }
@@ -223,17 +236,21 @@ template <> struct Deq<Q8_0> {
     {
         return row_ptr(w, 32, 2, 0, row);
     }
-    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int k0, int h)
+    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int s, int last, int h)
     {
-        const int blk = (k0 >> 5) + h;
-        r.a = *reinterpret_cast<const uint4 *>(p.p0 + blk * 32);
-        r.b = *reinterpret_cast<const uint4 *>(p.p0 + blk * 32 + 16);
-        r.d = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 2);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int blk = 2 * min(s + c, last) + h;
+            r.a[c] = *reinterpret_cast<const u32x4 *>(p.p0 + blk * 32);
+            r.b[c] = *reinterpret_cast<const u32x4 *>(p.p0 + blk * 32 + 16);
+            r.d[c] = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 2);
+        }
     }
-    __device__ __forceinline__ static void values(const Raw &r, int, int h, half8 (&w)[4])
+    __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
-        const float d = h2f(r.d), o = -128.f * d;
-        const uint32_t q[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+        const float d = h2f(r.d[u]), o = -128.f * d;
+        const u32x4 &a = r.a[u], &b = r.b[u];
+        const uint32_t q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) // q + 128
             w[i] = deq8(q[2 * i] ^ 0x80808080u, q[2 * i + 1] ^ 0x80808080u, d, o);
@@ -245,7 +262,7 @@ template <> struct Deq<Q8_0> {
 // half h takes k = 2h and 2h+1 (columns 32h..32h+31).
 template <> struct Deq<Q2_0C> {
     struct Raw {
-        uint4 c;
+        u32x4 c[4];
         uint32_t d;
     };
     __device__ static constexpr int c0(int h) { return 32 * h; }
@@ -254,16 +271,17 @@ template <> struct Deq<Q2_0C> {
     {
         return row_ptr(w, 128, 2, 0, row);
     }
-    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int k0, int)
+    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int s, int, int)
     {
-        const int blk = k0 >> 9, u = (k0 >> 6) & 7;
-        r.c = *reinterpret_cast<const uint4 *>(p.p0 + blk * 128 + u * 16);
-        r.d = *reinterpret_cast<const uint16_t *>(p.p1 + blk * 2);
+        r.d = *reinterpret_cast<const uint16_t *>(p.p1 + (s >> 3) * 2);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            r.c[c] = *reinterpret_cast<const u32x4 *>(p.p0 + (s + c) * 16);
     }
-    __device__ __forceinline__ static void values(const Raw &r, int, int h, half8 (&w)[4])
+    __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
         const float d = h2f(r.d), d2 = 2.f * d, o = -3.f * d;
-        const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
+        const uint32_t cw[4] = {r.c[u].x, r.c[u].y, r.c[u].z, r.c[u].w};
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -281,8 +299,8 @@ template <> struct Deq<Q2_0C> {
 // and their signs at bits (c%2)*4 + j + 8t of the chunk pair's sign dword.
 template <> struct Deq<STQ1_0> {
     struct Raw {
-        uint2 nib;
-        uint32_t s, d;
+        u32x4 nib[2];
+        uint32_t s[2], d;
     };
     __device__ static constexpr int c0(int h) { return 32 * h; }
     __device__ static constexpr int c1(int h) { return 32 * h + 16; }
@@ -290,23 +308,26 @@ template <> struct Deq<STQ1_0> {
     {
         return row_ptr(w, 32, 8, 2, row);
     }
-    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int k0, int)
+    __device__ __forceinline__ static void load(Raw &r, const RowPtr &p, int s, int, int)
     {
-        const int blk = k0 >> 8, c = (k0 >> 6) & 3;
-        r.nib = *reinterpret_cast<const uint2 *>(p.p0 + blk * 32 + 8 * c);
-        r.s = *reinterpret_cast<const uint32_t *>(p.p1 + blk * 8 + 4 * (c >> 1));
+        const int blk = s >> 2;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            r.nib[i] = *reinterpret_cast<const u32x4 *>(p.p0 + blk * 32 + 16 * i);
+            r.s[i] = *reinterpret_cast<const uint32_t *>(p.p1 + blk * 8 + 4 * i);
+        }
         r.d = *reinterpret_cast<const uint16_t *>(p.p2 + blk * 2);
     }
     __device__ __forceinline__ static void values(const Raw &r, int u, int h, half8 (&w)[4])
     {
         const int c = u;
         const float d = h2f(r.d), o = -d;
-        const uint32_t nb[2] = {r.nib.x, r.nib.y};
+        const uint32_t nb[2] = {r.nib[c >> 1][2 * (c & 1)], r.nib[c >> 1][2 * (c & 1) + 1]};
         uint32_t e[4]; // the groups' codebook entries, four per dword
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t nibs = (nb[j >> 1] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-            const uint32_t sb = ((r.s >> ((c & 1) * 4 + j)) & 0x01010101u) << 4;
+            const uint32_t sb = ((r.s[c >> 1] >> ((c & 1) * 4 + j)) & 0x01010101u) << 4;
             e[j] = GroupSTQ::lut(nibs | sb) >> (4 * h);
         }
 #pragma unroll
@@ -318,377 +339,198 @@ template <> struct Deq<STQ1_0> {
     }
 };
 
-// Zeros for LDS rows past the end of the weight (each half clears 32 columns).
-__device__ __forceinline__ void zero_half(_Float16 *dst, int h)
-{
-    const half8 z = {};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<half8 *>(dst + 32 * h + 8 * i) = z;
-}
-
-// ---------------------------------------------------------------------------
-// Activation slice: BN rows (tokens) x 64 f16 columns, 16 bytes per thread
-// per load: index f = t + 256 i -> row f/8 = t/8 + 32 i, columns 8*(t%8)...
-// xp[i] is the thread's row pointer for load i (offset by its 8 columns),
-// nullptr for rows past the end (zeros).
-// ---------------------------------------------------------------------------
-struct XRaw {
-    uint4 v[4];
-};
-
-__device__ __forceinline__ void load_x(XRaw &x, const _Float16 *const (&xp)[4], int k0)
-{
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        x.v[i] = xp[i] ? *reinterpret_cast<const uint4 *>(xp[i] + k0) : make_uint4(0, 0, 0, 0);
-}
-
-// NW waves: load i of thread t covers token row t / 8 + 8 NW i.
-template <int NW = 4> __device__ __forceinline__ void store_x(_Float16 *Xs, const XRaw &x)
-{
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint4 *>(Xs + ((t >> 3) + 8 * NW * i) * LDK + 8 * (t & 7)) = x.v[i];
-}
-
-// LDS halves of one operand buffer (weights, then activations) and of the
-// two buffers a k_loop of NW waves uses.
-template <int NW> constexpr int buf_halves() { return TILE_HALVES + 32 * NW * LDK; }
-template <int NW> constexpr int lds_halves() { return 2 * buf_halves<NW>(); }
-
-// One 64-deep step: acc[i][j] accumulates LDS weight rows arow(i) + lane%32
-// against tokens wn*64 + 32*j + lane%32, for the wave's first J token
-// blocks (the others hold no token of the tile).
-template <int J, class ARow>
-__device__ __forceinline__ void mma_step(const _Float16 *Ws, const _Float16 *Xs, const ARow &arow,
-                                         int wn, f32x16 (&acc)[2][2])
-{
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 31, kq = 8 * (lane >> 5);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-        half8 a[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            a[i] = *reinterpret_cast<const half8 *>(Ws + (arow(i) + r) * LDK + kk + kq);
-            if (i < J)
-                b[i] = *reinterpret_cast<const half8 *>(Xs + (wn * 64 + 32 * i + r) * LDK + kk +
-                                                        kq);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-}
-
 // v_mfma 32x32 output layout: register e of a block holds row
 // 8*(e/4) + 4*(lane/32) + e%4 and column lane%32 of the block.
 __device__ __forceinline__ int acc_row_in_block(int e)
 {
     return 8 * (e >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (e & 3);
 }
-__device__ __forceinline__ int acc_col(int wn, int j)
-{
-    return wn * 64 + 32 * j + (threadIdx.x & 31);
-}
-
-__device__ __forceinline__ void zero_acc(f32x16 (&acc)[2][2])
-{
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-}
-
 // ---------------------------------------------------------------------------
-// The K loop shared by every GEMM kernel. wsrc(lrow, view, row) sets the
-// weight view and row that LDS row lrow dequantizes (row < 0: zeros);
-// xrow(r) gives the f16 activation row of token r of the tile (nullptr =
-// zeros); arow(i) the first LDS weight row of the wave's block i. lds holds
-// lds_halves<NW>() halves: buffer b at lds + b * buf_halves<NW>(), weights
-// then activations. The loop covers columns [kbase, kbase + K) (a K slice
-// when kbase > 0; both multiples of the format's block). JM = 1 is the
-// variant for tiles of at most 32 tokens (MoE experts): only the first token
-// block holds tokens, so the waves with wn = 1 skip their MFMAs and the
-// others run one token block.
+// The K loop of every tile kernel: 512 threads, waves 0-3 (one per SIMD)
+// dequantize the weights, waves 4-7 (the other wave of each SIMD) multiply.
+//
+// LDS holds only the dequantized weights: two buffers of BM rows x BK columns.
+// The activations come in fragment order (hyq_f16rows.hpp) straight into the
+// consumers' registers, a contiguous KiB per load of a full 32-token block.
+// A shape C has NP = 4 producer and NC consumer waves, WR of which share the tokens and split the rows, each
+// holding C::RB row blocks by C::CB token blocks of 32 (WR = 1: 4 x 2 blocks,
+// a tile of 128 rows by 256 tokens, or RB = 3, 96, or RB = 2, 64 rows; WR = 2:
+// 2 x CB blocks, 128 rows by 64 CB tokens). Wave (wr, wc) takes the token blocks wc, wc + WC,
+// ..., and only those that hold tokens of the tile (cnt), so a partial tile
+// costs its own blocks. Per MFMA a wave reads 1/CB KiB from LDS and 1/RB from
+// L1/L2.
+//
+// What bounds it: the consumers' MFMAs and, where few token blocks share a
+// dequantized weight, the producers' conversion (about 3.2 VALU instructions
+// per weight). Both are kept from waiting:
+//  - the packed bytes of the next four steps are in flight in the producers'
+//    registers;
+//  - the consumers are software-pipelined, held by scheduling barriers: the
+//    weight fragments of the next 16 columns are read from LDS before the
+//    current ones' MFMAs (the compiler else keeps two in flight, each pair
+//    of MFMAs waiting for its own), the tokens NS steps ahead into the
+//    registers just consumed (unconditionally, past the end the last step
+//    again: a branch there made every other step wait for the loads it had
+//    just issued);
+//  - a step's buffer is done with once its last fragments are in registers,
+//    so its barrier comes before their MFMAs and the next buffer's first reads
+//    run under them.
+//
+// wsrc(lrow, view, row): the weight view and row that LDS row lrow
+// dequantizes (any of the view's for a row past the end, whose sums nobody
+// writes); xt: the operand run of the tile's first
+// token, cnt >= 1 its tokens; arow(i): the first LDS row of the wave's row
+// block i. The loop covers columns [kbase, kbase + klen) of K (multiples of
+// the format's block and of BK). Every output element sees the same operands
+// in the same k order in every form: bit-identical results.
 // ---------------------------------------------------------------------------
-template <int F, int JM = 2, int NW = 4, class WSrc, class XRow, class ARow>
-__device__ __forceinline__ void k_loop(const WSrc &wsrc, const XRow &xrow, const ARow &arow,
-                                       int K, int wn, _Float16 *lds, f32x16 (&acc)[2][2],
-                                       int kbase = 0)
-{
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    using D = Deq<F>;
-    constexpr int BUF = buf_halves<NW>();
-    const int t = threadIdx.x;
-    // the first 256 threads dequantize the weight slice (a wave-uniform test)
-    const bool wthr = NW == 4 || t < 256;
-    const int lrow = (t & 255) >> 1, h = t & 1;
-    WView wv{};
-    int row = -1;
-    wsrc(lrow, wv, row);
-    const RowPtr rp = D::rows(wv, row < 0 ? 0 : row);
-    const _Float16 *xp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const _Float16 *p = xrow((t >> 3) + 8 * NW * i);
-        xp[i] = p ? p + 8 * (t & 7) : nullptr;
-    }
-    typename D::Raw raw;
-    XRaw xr;
-    auto fetch = [&](int k0) {
-        if (wthr && row >= 0) D::load(raw, rp, kbase + k0, h);
-        load_x(xr, xp, kbase + k0);
-    };
-    auto put = [&](int k0, int b) {
-        _Float16 *Ws = lds + b * BUF;
-        if (wthr) {
-            if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
-            else zero_half(Ws + lrow * LDK, h);
-        }
-        store_x<NW>(Ws + TILE_HALVES, xr);
-    };
-    const int steps = K / BK;
-    const bool mma = JM == 2 || __builtin_amdgcn_readfirstlane(wn) == 0;
-    fetch(0);
-    put(0, 0);
-    if (steps > 1) fetch(BK);
-    __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-        const int cur = s & 1;
-        const _Float16 *Ws = lds + cur * BUF;
-        if (mma) mma_step<JM>(Ws, Ws + TILE_HALVES, arow, wn, acc);
-        if (s + 1 < steps) {
-            put((s + 1) * BK, cur ^ 1);
-            if (s + 2 < steps) fetch((s + 2) * BK);
-        }
-        __syncthreads();
-    }
-}
+constexpr int PX_LDS = 2 * TILE_HALVES;
 
-// ---------------------------------------------------------------------------
-// Producer/consumer form of k_loop for 512 threads (tiles of BM weight rows by
-// 256 tokens): waves 0-3 (one per SIMD) fetch and dequantize the weight slice
-// as k_loop's first 256 threads do; waves 4-7 (the other wave of each SIMD)
-// multiply, each 2 blocks of 32 weight rows (LDS rows arow(0), arow(1) ..
-// + 31, a function of the wave) by 128 tokens, wave 4 + c taking tokens
-// 128 (c % 2): 2 weight and 4 token fragments per 16-deep step feed 8
-// MFMAs (0.75 KB of LDS reads per MFMA against k_loop's 1 KB); all eight
-// copy the activation slice as k_loop does (four 16-byte pieces each). Every output
-// element sees the same operands in the same k order as in k_loop, so the
-// results are bit-identical. acc[i][j]: weight block i, token block j.
-// ---------------------------------------------------------------------------
-constexpr int PC_THREADS = 512;
-
-template <class ARow>
-__device__ __forceinline__ void mma_step_pc(const _Float16 *Ws, const _Float16 *Xs,
-                                            const ARow &arow, int wn, f32x16 (&acc)[2][4])
-{
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 31, kq = 8 * (lane >> 5);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-        half8 a[2], b[4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            a[i] = *reinterpret_cast<const half8 *>(Ws + (arow(i) + r) * LDK + kk + kq);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            b[j] = *reinterpret_cast<const half8 *>(Xs + (wn * 128 + 32 * j + r) * LDK + kk + kq);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-}
-
-template <int F, class WSrc, class XRow, class ARow>
-__device__ __forceinline__ void k_loop_pc(const WSrc &wsrc, const XRow &xrow, const ARow &arow,
-                                          int K, _Float16 *lds, f32x16 (&acc)[2][4],
-                                          int kbase = 0)
+template <int F, int ROWS, int PART, class WSrc>
+__device__ __forceinline__ void px_produce(const WSrc &wsrc, int steps, int kbase, _Float16 *lds)
 {
     using D = Deq<F>;
-    constexpr int BUF = buf_halves<8>();
-    const int t = threadIdx.x;
-    // waves 0-3 produce, waves 4-7 consume (a wave-uniform test); both copy
-    // activation rows: thread t the four rows (t % 256) / 8 + 32 i + 128 (t / 256)
-    const bool prod = __builtin_amdgcn_readfirstlane(t) < 256;
-    const int lrow = (t & 255) >> 1, h = t & 1;
-    const int wn = (t >> 6) & 1;
-    WView wv{};
-    int row = -1;
-    if (prod) wsrc(lrow, wv, row);
-    const _Float16 *xp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const _Float16 *p = xrow(((t & 255) >> 3) + 32 * i + 128 * (t >> 8));
-        xp[i] = p ? p + 8 * (t & 7) : nullptr;
-    }
-    const RowPtr rp = D::rows(wv, row < 0 ? 0 : row);
-    typename D::Raw raw;
-    uint4 xr[4];
-    auto fetch_x = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            xr[i] = xp[i] ? *reinterpret_cast<const uint4 *>(xp[i] + kbase + k0)
-                          : make_uint4(0, 0, 0, 0);
-    };
-    auto put_x = [&](int b) {
-        _Float16 *Xs = lds + b * BUF + TILE_HALVES;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<uint4 *>(
-                Xs + (((t & 255) >> 3) + 32 * i + 128 * (t >> 8)) * LDK + 8 * (t & 7)) = xr[i];
-    };
-    auto fetch_w = [&](int k0) {
-        if (row >= 0) D::load(raw, rp, kbase + k0, h);
-    };
-    auto put_w = [&](int k0, int b) {
-        _Float16 *Ws = lds + b * BUF;
-        if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws + lrow * LDK);
-        else zero_half(Ws + lrow * LDK, h);
-    };
-    // Two loops, one per role, each passing the same 1 + steps barriers (a
-    // barrier counts waves, whichever instruction they reach it at), so that
-    // neither role keeps the other's registers live: the producers' staged
-    // weights, the consumers' 128 accumulators.
-    const int steps = K / BK;
-    if (prod) {
-        fetch_w(0);
-        fetch_x(0);
-        put_w(0, 0);
-        put_x(0);
-        if (steps > 1) {
-            fetch_w(BK);
-            fetch_x(BK);
-        }
-        __syncthreads();
-        for (int s = 0; s < steps; ++s) {
-            if (s + 1 < steps) {
-                put_w((s + 1) * BK, (s & 1) ^ 1);
-                put_x((s & 1) ^ 1);
-                if (s + 2 < steps) {
-                    fetch_w((s + 2) * BK);
-                    fetch_x((s + 2) * BK);
-                }
-            }
-            __syncthreads();
-        }
-    } else {
-        fetch_x(0);
-        put_x(0);
-        if (steps > 1) fetch_x(BK);
-        __syncthreads();
-        for (int s = 0; s < steps; ++s) {
-            const _Float16 *Ws = lds + (s & 1) * BUF;
-            mma_step_pc(Ws, Ws + TILE_HALVES, arow, wn, acc);
-            if (s + 1 < steps) {
-                put_x((s & 1) ^ 1);
-                if (s + 2 < steps) fetch_x((s + 2) * BK);
-            }
-            __syncthreads();
-        }
-    }
-}
-
-// The producer/consumer loop with the activations, in fragment order
-// (launch_to_f16 with frag), taken straight into the consumers' registers (no
-// LDS copy): consumer wave 4 + c owns tokens 64 c .. 64 c + 63 of the tile
-// against all 32 NI weight rows (NI weight and 2 token fragments per 16-deep
-// step feed 2 NI MFMAs), loading its token fragments one step ahead into a
-// two-set register ring, each a contiguous KiB (lane l: 8 consecutive k of
-// token 32 j + l % 32); LDS holds only the dequantized weights. NI = 4 is
-// the 128-row tile; NI = 3 a 96-row tile (producer threads of rows 96-127
-// idle), for grids that 128-row tiles would leave short of the CUs.
-// xsrc(r): the fragment-order run of the 32-token block of tile token r
-// (clamped into the batch: tokens past it produce sums nobody writes). Same
-// operands, same k order per element as k_loop: bit-identical results.
-// acc[i][j]: weight block i, token block j.
-template <int F, int NI, class WSrc, class XSrc>
-__device__ __forceinline__ void k_loop_pcx(const WSrc &wsrc, const XSrc &xsrc, int K,
-                                           _Float16 *lds, f32x16 (&acc)[NI][2], int kbase = 0)
-{
-    static_assert(NI == 3 || NI == 4, "96- or 128-row tiles");
-    using D = Deq<F>;
-    const int t = threadIdx.x;
-    const bool prod = __builtin_amdgcn_readfirstlane(t) < 256;
-    const int steps = K / BK;
-    if (prod) {
-        const int lrow = t >> 1, h = t & 1;
-        const bool used = lrow < 32 * NI;
-        WView wv{};
-        int row = -1;
-        if (used) wsrc(lrow, wv, row);
-        const RowPtr rp = D::rows(wv, row < 0 ? 0 : row);
-        typename D::Raw raw;
-        auto fetch = [&](int k0) {
-            if (row >= 0) D::load(raw, rp, kbase + k0, h);
-        };
-        auto put = [&](int k0, int b) {
-            _Float16 *Ws = lds + b * TILE_HALVES + lrow * LDK;
-            if (row >= 0) convert<F>(raw, ((kbase + k0) >> 6) & 3, h, Ws);
-            else if (used) zero_half(Ws, h);
-        };
-        fetch(0);
-        put(0, 0);
-        if (steps > 1) fetch(BK);
-        __syncthreads();
-        for (int s = 0; s < steps; ++s) {
-            if (s + 1 < steps) {
-                put((s + 1) * BK, (s & 1) ^ 1);
-                if (s + 2 < steps) fetch((s + 2) * BK);
-            }
-            __syncthreads();
-        }
+    // (64 rows: two threads to a weight's 32 columns, one per PART)
+    const int t = threadIdx.x & (ROWS > 64 ? 255 : 127), lrow = t >> 1, h = t & 1;
+    if (ROWS < BM && __builtin_amdgcn_readfirstlane(lrow) >= ROWS) { // (by wave)
+        for (int s = 0; s <= steps; ++s) __syncthreads();
         return;
     }
-    const int lane = t & 63, c = (t >> 6) & 3;
-    const int r = lane & 31, kq = 8 * (lane >> 5);
-    // lane l's 8 halves of 16-deep step b in the block's fragment-order run
-    const _Float16 *xb[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) xb[j] = xsrc(64 * c + 32 * j) + (size_t)(kbase / 16) * 512 + lane * 8;
-    half8 B0[4][2], B1[4][2];
-    auto loadB = [&](half8 (&b)[4][2], int k0) {
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                b[kk][j] = *reinterpret_cast<const half8 *>(xb[j] + (size_t)(k0 / 16 + kk) * 512);
+    WView wv{};
+    int row = 0;
+    wsrc(lrow, wv, row);
+    const RowPtr rp = D::rows(wv, row);
+    // two 256-column blocks: one is dequantized while the next is loaded (the
+    // last again, unused, past the end), in straight-line code: a load under
+    // a condition, or a loop left in its middle and entered again, makes the
+    // compiler's counted waits wait for the loads just issued
+    typename D::Raw raw[2];
+    const int s0 = kbase / BK, blocks = (steps + 3) / 4;
+    auto fetch = [&](int b, int i) {
+        D::load(raw[i], rp, s0 + 4 * min(b, blocks - 1), s0 + steps - 1, h);
     };
-    auto mma = [&](const _Float16 *Ws, const half8 (&b)[4][2]) {
+    fetch(0, 0);
+    for (int bb = 0;; bb += 2) {
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            half8 a[NI];
+        for (int i = 0; i < 2; ++i) {
+            fetch(bb + i + 1, i ^ 1);
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
-                a[i] = *reinterpret_cast<const half8 *>(Ws + (32 * i + r) * LDK + 16 * kk + kq);
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] =
-                        __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[kk][j], acc[i][j], 0, 0, 0);
-        }
-    };
-    loadB(B0, 0);
-    __syncthreads();
-    for (int s = 0; s < steps; s += 2) {
-        if (s + 1 < steps) loadB(B1, (s + 1) * BK);
-        mma(lds, B0);
-        __syncthreads();
-        if (s + 1 < steps) {
-            if (s + 2 < steps) loadB(B0, (s + 2) * BK);
-            mma(lds + TILE_HALVES, B1);
-            __syncthreads();
+            for (int u = 0; u < 4; ++u) {
+                convert<F, PART>(raw[i], u, h, lds + (u & 1) * TILE_HALVES + lrow * LDK);
+                __syncthreads();
+                // (only Q8_0's rows may end within a block)
+                if ((u == 3 || F == Q8_0) && 4 * (bb + i) + u + 1 >= steps) {
+                    __syncthreads();
+                    return;
+                }
+            }
         }
     }
+}
+
+template <int RB, int CB, int J, int NS, class ARow>
+__device__ __forceinline__ void px_consume(const _Float16 *xt, int cnt, int K, int wc, int WC,
+                                           const ARow &arow, int steps, int kbase,
+                                           const _Float16 *lds, f32x16 (&acc)[RB][CB])
+{
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    const _Float16 *xb[J];
+    unsigned stride[J]; // halves per 16 columns of the block
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int b = j * WC + wc, c = min(32, cnt - 32 * b);
+        xb[j] = xt + (size_t)32 * b * K + (size_t)kbase * c + (h * c + min(r, c - 1)) * 8;
+        stride[j] = 16 * c;
+    }
+    half8 B[NS][4][J], a[2][RB];
+    auto loadB = [&](int s, int set, int kk) {
+        const unsigned k16 = 4u * min(s, steps - 1) + kk;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+            B[set][kk][j] = *reinterpret_cast<const half8 *>(xb[j] + k16 * stride[j]);
+    };
+    auto loadA = [&](int set, const _Float16 *Ws, int kk) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+            a[set][i] = *reinterpret_cast<const half8 *>(Ws + (arow(i) + r) * LDK + 16 * kk + 8 * h);
+    };
+#pragma unroll
+    for (int p = 0; p < NS; ++p)
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            loadB(p, p, kk);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    __syncthreads();
+    loadA(0, lds, 0);
+    auto step = [&](int s, int p) {
+        const _Float16 *Ws = lds + p * TILE_HALVES, *Wn = lds + (p ^ 1) * TILE_HALVES;
+        const int set = p & (NS - 1);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            if (kk < 3) {
+                loadA((kk + 1) & 1, Ws, kk + 1);
+            } else {
+                __syncthreads();
+                loadA(0, Wn, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kk & 1][i], B[set][kk][j],
+                                                                       acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            loadB(s + NS, set, kk);
+        }
+    };
+    int s = 0;
+    for (; s + 1 < steps; s += 2) {
+        step(s, 0);
+        step(s + 1, 1);
+    }
+    if (s < steps) step(s, 0);
+}
+
+// acc[i][j]: row block arow(i), token block j * WC + wc of the tile. Returns
+// false for the producers, which hold no sums.
+template <int F, class C, class WSrc, class ARow>
+__device__ __forceinline__ bool k_loop_px(const WSrc &wsrc, const ARow &arow, const _Float16 *xt,
+                                          int cnt, int K, int kbase, int klen, _Float16 *lds,
+                                          f32x16 (&acc)[C::RB][C::CB])
+{
+    constexpr int RB = C::RB, CB = C::CB, NS = C::NS, WC = C::NC / C::WR;
+    static_assert(32 * C::WR * RB <= BM && NS >= 1 && NS <= 2 && CB <= 3 &&
+                      C::NP == 4,
+                  "tile shape");
+    const int steps = klen / BK, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wave < C::NP) {
+        constexpr int ROWS = 32 * C::WR * RB;
+        if (ROWS > 64) px_produce<F, ROWS, -1>(wsrc, steps, kbase, lds);
+        else if (wave < 2) px_produce<F, ROWS, 0>(wsrc, steps, kbase, lds);
+        else px_produce<F, ROWS, 1>(wsrc, steps, kbase, lds);
+        return false;
+    }
+    const int wc = (wave - C::NP) % WC;
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    // this wave's token blocks; both roles pass 1 + steps barriers
+    const int nj = ((cnt + 31) / 32 - wc + WC - 1) / WC;
+    if (nj >= CB) {
+        px_consume<RB, CB, CB, NS>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
+    } else if (CB > 2 && nj == 2) {
+        px_consume<RB, CB, 2 < CB ? 2 : 1, NS>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
+    } else if (CB > 1 && nj == 1) {
+        px_consume<RB, CB, 1, NS>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
+    } else {
+        for (int s = 0; s <= steps; ++s) __syncthreads();
+    }
+    return true;
 }
 
 } // namespace tile

@@ -255,3 +255,45 @@ def test_register_operand_products(gpu_ctx, hyq, oracle, dtype, rows, cols):
         assert np.array_equal(y[:top * rows].reshape(top, rows), full)
         assert np.all(y[top * rows:] == 5.0)
     W.release()
+
+
+@pytest.mark.parametrize("dtype", QUANT, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("rows,cols", [(200, 1024), (130, 2560)], ids=["200x1024", "130x2560"])
+def test_tile_shapes_at_block_edges(gpu_ctx, oracle, dtype, rows, cols):
+    """Token counts on both sides of every tile shape (128, 192 and 256 tokens)
+    and of a wave's token blocks, rows that end inside a tile: parity with the
+    oracle, which is token-local; on one side of 128 tokens (the K split's
+    classes) a token's row has the same bits at any count."""
+    _print("tile shapes", NAMES[dtype], rows, cols)
+    w = random_matrix(dtype, rows, cols, seed=rows + dtype)
+    top = 520
+    x = np.random.default_rng(cols + dtype).normal(0, 1, top * cols).astype(np.float32)
+    y_ref, mag = oracle.matmul_f64(dtype, w, rows, cols, x, top)
+    y_ref, mag = y_ref.reshape(top, rows), mag.reshape(top, rows)
+    W = gpu_ctx.upload(dtype, w, (cols, rows))
+    seen = {}
+    for batch in (65, 96, 97, 128, 129, 160, 161, 192, 193, 225, 256, 257, 385, 513, top):
+        y = W.matmul(x[:batch * cols], batch).reshape(batch, rows)
+        check_prefill_path(y, y_ref[:batch], mag[:batch], f"{NAMES[dtype]} batch {batch}")
+        kind = batch > 128
+        n = min(batch, len(seen.get(kind, y)))
+        assert np.array_equal(y[:n], seen.get(kind, y)[:n]), batch
+        seen[kind] = y
+    W.release()
+
+
+@pytest.mark.parametrize("cols", [64, 192, 576, 1088])
+@pytest.mark.parametrize("batch", [3, 70, 140, 300])
+def test_q80_rows_ending_inside_a_set(gpu_ctx, oracle, cols, batch):
+    """Q8_0 rows of 1, 3, 9 and 17 64-column steps: the last set of four loads
+    its missing steps clamped to the row's end (the weight's last row included)
+    and an odd last step runs alone."""
+    rows = 140
+    _print("q80 partial set", cols, batch)
+    w = random_matrix(Q8_0, rows, cols, seed=cols)
+    x = np.random.default_rng(cols + batch).normal(0, 1, batch * cols).astype(np.float32)
+    W = gpu_ctx.upload(Q8_0, w, (cols, rows))
+    y = W.matmul(x, batch).reshape(batch, rows)
+    y_ref, mag = oracle.matmul_f64(Q8_0, w, rows, cols, x, batch)
+    check_prefill_path(y, y_ref.reshape(batch, rows), mag.reshape(batch, rows), f"cols {cols}")
+    W.release()
