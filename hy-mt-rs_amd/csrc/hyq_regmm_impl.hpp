@@ -129,7 +129,6 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
         };
         // (straight-line blocks left only at the loop's end: see px_produce)
         auto block = [&](int d, int b, int n) {
-            load_w(d ^ 1, b + 1);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 if (F == Q8_0 && u >= n) return;
@@ -147,9 +146,11 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
                                                                             acc[b], 0, 0, 0);
                     if (s == 0) load_b(0, min(c + 1, c1 - 1));
                 }
+                if (u == 3) load_w(d, b + 2);
             }
         };
         load_w(0, b0);
+        load_w(1, b0 + 1);
         load_b(0, c0);
         for (int b = b0;; b += 2) {
             block(0, b, c1 - 4 * b);
