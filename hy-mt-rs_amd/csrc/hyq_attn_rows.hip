@@ -290,31 +290,59 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const float *__restrict
     float *den = wt + heads * splits; // [heads]
     const int nact = min((*pos_p + tq + chunk) / chunk, splits);
     const float *pt = part + (size_t)tq * heads * splits * PART_STRIDE;
+    // every (head, split)'s maximum and exp-sum in one pass of loads (the
+    // exp-sums where the row comes later: splits <= 128 of them per head)
+    for (int i = t; i < heads * nact; i += 256) {
+        const int h = i / nact, sp = i - h * nact;
+        const float2 ml =
+            *reinterpret_cast<const float2 *>(pt + ((size_t)h * splits + sp) * PART_STRIDE);
+        wt[h * splits + sp] = ml.x;
+        row[h * splits + sp] = ml.y;
+    }
+    __syncthreads();
     for (int h = t; h < heads; h += 256) {
-        const float *ph = pt + (size_t)h * splits * PART_STRIDE;
         float M = -INFINITY;
-        for (int sp = 0; sp < nact; ++sp) M = fmaxf(M, ph[(size_t)sp * PART_STRIDE]);
+        for (int sp = 0; sp < nact; ++sp) M = fmaxf(M, wt[h * splits + sp]);
+        den[h] = M;
+    }
+    __syncthreads();
+    for (int i = t; i < heads * nact; i += 256) {
+        const int h = i / nact, sp = i - h * nact;
+        wt[h * splits + sp] = expf(wt[h * splits + sp] - den[h]);
+    }
+    __syncthreads();
+    for (int h = t; h < heads; h += 256) {
         float d = 0.f;
-        for (int sp = 0; sp < nact; ++sp) {
-            const float w = expf(ph[(size_t)sp * PART_STRIDE] - M);
-            wt[h * splits + sp] = w;
-            d += w * ph[(size_t)sp * PART_STRIDE + 1];
-        }
+        for (int sp = 0; sp < nact; ++sp) d += wt[h * splits + sp] * row[h * splits + sp];
         den[h] = d;
     }
     __syncthreads();
     float mx = 0.f;
-    for (int i = t; i < W; i += 256) {
-        const int h = i / ATT_D, dd = i % ATT_D;
+    for (int i = t; i < W / 4; i += 256) {
+        const int h = i / (ATT_D / 4), dd = 4 * (i % (ATT_D / 4));
         const float *ph = pt + (size_t)h * splits * PART_STRIDE + 4 + dd;
-        float num = 0.f;
-#pragma unroll 4
-        for (int sp = 0; sp < nact; ++sp) num += wt[h * splits + sp] * ph[(size_t)sp * PART_STRIDE];
-        const float v = num / den[h];
-        row[i] = v;
-        if (out) out[(size_t)tq * W + i] = v;
-        mx = fmaxf(mx, fabsf(v));
-        if (v != v) mx = INFINITY;
+        float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 8
+        for (int sp = 0; sp < nact; ++sp) {
+            const float w = wt[h * splits + sp];
+            const float4 p = *reinterpret_cast<const float4 *>(ph + (size_t)sp * PART_STRIDE);
+            num.x += w * p.x;
+            num.y += w * p.y;
+            num.z += w * p.z;
+            num.w += w * p.w;
+        }
+        const float d = den[h];
+        const float4 v = make_float4(num.x / d, num.y / d, num.z / d, num.w / d);
+        reinterpret_cast<float4 *>(row)[i] = v;
+        if (out) { // (the caller's, 4-byte aligned)
+            float *o = out + (size_t)tq * W + 4 * i;
+            o[0] = v.x;
+            o[1] = v.y;
+            o[2] = v.z;
+            o[3] = v.w;
+        }
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        if (v.x != v.x || v.y != v.y || v.z != v.z || v.w != v.w) mx = INFINITY;
     }
     if (!xh) return;
     __shared__ float red[4];
@@ -327,7 +355,12 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const float *__restrict
     if (t == 0) rscale[tq] = ldexpf(1.0f, e);
     const int first = tq & ~31, bt = min(32, (int)gridDim.x - first);
     _Float16 *o = xh + (size_t)first * W;
-    for (int i = t; i < W; i += 256) o[frag_at(i, tq - first, bt)] = (_Float16)(row[i] * inv);
+    for (int i = t; i < W / 4; i += 256) {
+        const float4 v = reinterpret_cast<const float4 *>(row)[i];
+        const half4 r = {(_Float16)(v.x * inv), (_Float16)(v.y * inv), (_Float16)(v.z * inv),
+                         (_Float16)(v.w * inv)};
+        *reinterpret_cast<half4 *>(o + frag_at(4 * i, tq - first, bt)) = r;
+    }
 }
 
 } // namespace

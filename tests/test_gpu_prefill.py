@@ -64,6 +64,25 @@ def test_attention_rows_matches_oracle(gpu_ctx, hyq, oracle, pos, n, heads, kvh)
         assert np.allclose(got[i], ref, rtol=1e-5, atol=1e-6), (i, np.abs(got[i] - ref).max())
 
 
+@pytest.mark.parametrize("heads,kvh,ctxlen,pos,n", [(64, 16, 9000, 8990, 9), (4, 4, 130, 0, 130),
+                                                    (48, 16, 1024, 120, 17)])
+def test_attention_merge_of_many_splits(gpu_ctx, hyq, oracle, heads, kvh, ctxlen, pos, n):
+    """The row merge at its widest split count (60 splits of 64 heads), at one
+    and two splits, and at rows of 24 waves' worth of heads."""
+    D = 128
+    _print("attention merge", heads, kvh, ctxlen, pos, n)
+    rng = np.random.default_rng(heads + n)
+    q = rng.normal(0, 1, (n, heads * D)).astype(np.float32)
+    kc = rng.normal(0, 1, (ctxlen, kvh * D)).astype(np.float32)
+    vc = rng.normal(0, 1, (ctxlen, kvh * D)).astype(np.float32)
+    got = _attention_rows(hyq, gpu_ctx, q, kc, vc, pos, n, heads, kvh)
+    for i in range(0, n, 8):
+        ref = np.empty(heads * D, np.float32)
+        oracle.lib().hyqo_attention(q[i].ctypes.data, kc.ctypes.data, vc.ctypes.data, heads,
+                                    kvh, D, pos + i + 1, ref.ctypes.data)
+        assert np.allclose(got[i], ref, rtol=1e-5, atol=1e-6), (i, np.abs(got[i] - ref).max())
+
+
 def test_attention_rows_do_not_see_future_values(gpu_ctx, hyq):
     """src/model.rs:1104-1125 at head_dim 128: zero queries and keys, two
     rows at positions 0 and 1 average the values they can see."""
