@@ -912,10 +912,13 @@ __global__ __launch_bounds__(tile_threads<TileMoe>(), TileMoe::OCC) void moe_gat
     int mtiles, int max_tiles)
 {
     __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
-    const int T = xcd_tile(mtiles * max_tiles);
-    if (T >= mtiles * max_tiles) return;
+    // (ranges of the tiles there are, not of the grid's bound: at 500 tokens of
+    // 64 experts those are 64 of 96, which left the last XCDs without work)
+    const int total = mtiles * min(*ntiles, max_tiles), per = (total + 7) / 8;
+    if ((int)(blockIdx.x / 8) >= per) return;
+    const int T = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (T >= total) return;
     const int ti = T / mtiles, mt = T % mtiles;
-    if (ti >= *ntiles) return;
     const int e = tiles[2 * ti], c = tiles[2 * ti + 1];
     const int nb = eoff[e] + c * BN;
     gate_up_tile<F, TileMoe>(gate, up, (size_t)e * mid, mid, mt * 64, K, xg + (size_t)nb * K,
@@ -946,10 +949,13 @@ __global__ __launch_bounds__(tile_threads<TileMoe>(), TileMoe::OCC) void moe_dow
 {
     using C = TileMoe;
     __shared__ __attribute__((aligned(16))) _Float16 lds[PX_LDS];
-    const int T = xcd_tile(mtiles * max_tiles);
-    if (T >= mtiles * max_tiles) return;
+    // (ranges of the tiles there are, not of the grid's bound: at 500 tokens of
+    // 64 experts those are 64 of 96, which left the last XCDs without work)
+    const int total = mtiles * min(*ntiles, max_tiles), per = (total + 7) / 8;
+    if ((int)(blockIdx.x / 8) >= per) return;
+    const int T = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (T >= total) return;
     const int ti = T / mtiles, mt = T % mtiles;
-    if (ti >= *ntiles) return;
     const int e = tiles[2 * ti], c = tiles[2 * ti + 1];
     const int nb = eoff[e] + c * BN;
     const int cnt = min(BN, eoff[e + 1] - nb);

@@ -464,7 +464,7 @@ __device__ __forceinline__ void px_consume(const _Float16 *xt, int cnt, int K, i
     __syncthreads();
     loadA(0, lds, 0);
     auto step = [&](int s, int p) {
-        const _Float16 *Ws = lds + p * TILE_HALVES, *Wn = lds + (p ^ 1) * TILE_HALVES;
+        const _Float16 *Ws = lds + (p & 1) * TILE_HALVES, *Wn = lds + (p & 1 ^ 1) * TILE_HALVES;
         const int set = p & (NS - 1);
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
@@ -485,12 +485,16 @@ __device__ __forceinline__ void px_consume(const _Float16 *xt, int cnt, int K, i
             loadB(s + NS, set, kk);
         }
     };
+    // (U steps a round, by the rings of both; the last ones singly)
+    constexpr int U = NS > 2 ? NS : 2;
     int s = 0;
-    for (; s + 1 < steps; s += 2) {
-        step(s, 0);
-        step(s + 1, 1);
+    for (; s + U <= steps; s += U) {
+#pragma unroll
+        for (int d = 0; d < U; ++d) step(s + d, d);
     }
-    if (s < steps) step(s, 0);
+#pragma unroll
+    for (int d = 0; d + 1 < U; ++d)
+        if (s + d < steps) step(s + d, d);
 }
 
 // acc[i][j]: row block arow(i), token block j * WC + wc of the tile. Returns
@@ -526,7 +530,9 @@ __device__ __forceinline__ bool k_loop_px(const WSrc &wsrc, const ARow &arow, co
     } else if (CB > 2 && nj == 2) {
         px_consume<RB, CB, 2 < CB ? 2 : 1, NS>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
     } else if (CB > 1 && nj == 1) {
-        px_consume<RB, CB, 1, NS>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
+        // (one block leaves the registers for four steps ahead, and its steps,
+        // of half the MFMAs or less, need them)
+        px_consume<RB, CB, 1, 4>(xt, cnt, K, wc, WC, arow, steps, kbase, lds, acc);
     } else {
         for (int s = 0; s <= steps; ++s) __syncthreads();
     }
