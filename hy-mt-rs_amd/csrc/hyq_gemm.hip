@@ -854,12 +854,6 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
         }
 }
 
-__device__ __forceinline__ float silu_mul(float g, float u)
-{
-    // (g / (1 + exp(-g))) * u, DenseFfn::forward (src/model.rs:680-682)
-    return (g / (1.0f + expf(-g))) * u;
-}
-
 // Gate and up of a tile: the first half of the LDS rows (64; 32 for Tile64)
 // dequantizes gate rows m0 .., the second the same rows of up; the first half of a wave's row blocks is
 // gate, the second the matching up rows, so the SiLU product pairs registers

@@ -228,6 +228,9 @@ bool regmm_fits(int fmt, int cols, int batch);
 int regmm_kslices(int rows, int cols);
 int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale, int batch,
                  float *y, const float *residual, void *stream, int kslices, float *part);
+// h[batch][gate.rows] = silu(gate . x) * (up . x), the same shapes and operand.
+int launch_regmm_gate_up(int fmt, WView gate, WView up, int cols, const _Float16 *xh,
+                         const float *rscale, int batch, float *h, void *stream);
 
 // Byte offsets of the MoE scratch regions (hyq_gemm.hip: moe_layout).
 struct MoeLayout {

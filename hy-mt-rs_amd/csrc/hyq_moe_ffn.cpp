@@ -213,12 +213,20 @@ int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, const 
                "route");
     // output = shared.forward(input, n) (:699): two products, silu(g) * u, down
     HYQ_LAUNCH(launch_to_f16(xn, n, H, b.xh, b.rs, st), "to_f16");
-    HYQ_LAUNCH(launch_gate_up_f16(f.sgate->dtype, f.sgate->view, f.sup->view, H, b.xh, b.rs, n,
-                                  b.h, st),
+    // (few tokens: the register-operand products, whose workgroups of 32 rows
+    // reach more CUs than the tiles of so few rows)
+    HYQ_LAUNCH(regmm_fits(f.sgate->dtype, H, n)
+                   ? launch_regmm_gate_up(f.sgate->dtype, f.sgate->view, f.sup->view, H, b.xh,
+                                          b.rs, n, b.h, st)
+                   : launch_gate_up_f16(f.sgate->dtype, f.sgate->view, f.sup->view, H, b.xh, b.rs,
+                                        n, b.h, st),
                "moe_shared_gate_up");
     HYQ_LAUNCH(launch_to_f16(b.h, n, f.smid, b.xh, b.rs, st), "to_f16");
-    HYQ_LAUNCH(launch_gemm_f16(f.sdown->dtype, f.sdown->view, f.smid, b.xh, b.rs, n, b.ffo,
-                               nullptr, st),
+    HYQ_LAUNCH(regmm_fits(f.sdown->dtype, f.smid, n)
+                   ? launch_regmm(f.sdown->dtype, f.sdown->view, f.smid, b.xh, b.rs, n, b.ffo,
+                                  nullptr, st, 1, nullptr)
+                   : launch_gemm_f16(f.sdown->dtype, f.sdown->view, f.smid, b.xh, b.rs, n, b.ffo,
+                                     nullptr, st),
                "moe_shared_down");
     // the experts, added per token in ascending expert order (:700-722)
     HYQ_LAUNCH(launch_moe(f.gate->dtype, f.down->dtype, f.gate->view, f.up->view, f.down->view, H,

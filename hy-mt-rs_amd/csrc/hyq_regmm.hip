@@ -42,6 +42,18 @@ int regmm_kslices(int rows, int cols)
     return ks;
 }
 
+static int launch_format(int fmt, const regmm::Args &a, int tb, void *stream)
+{
+    switch (fmt) {
+    case Q2_0C: return launch_regmm_format<Q2_0C>(a, tb, stream);
+    case STQ1_0: return launch_regmm_format<STQ1_0>(a, tb, stream);
+    case Q4_K: return launch_regmm_format<Q4_K>(a, tb, stream);
+    case Q6_K: return launch_regmm_format<Q6_K>(a, tb, stream);
+    case Q8_0: return launch_regmm_format<Q8_0>(a, tb, stream);
+    default: return (int)hipErrorInvalidValue;
+    }
+}
+
 int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale, int batch,
                  float *y, const float *residual, void *stream, int kslices, float *part)
 {
@@ -62,17 +74,31 @@ int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rs
     a.xh = xh;
     a.rscale = rscale;
     a.part = part;
-    int rc = (int)hipErrorInvalidValue;
-    switch (fmt) {
-    case Q2_0C: rc = launch_regmm_format<Q2_0C>(a, tb, stream); break;
-    case STQ1_0: rc = launch_regmm_format<STQ1_0>(a, tb, stream); break;
-    case Q4_K: rc = launch_regmm_format<Q4_K>(a, tb, stream); break;
-    case Q6_K: rc = launch_regmm_format<Q6_K>(a, tb, stream); break;
-    case Q8_0: rc = launch_regmm_format<Q8_0>(a, tb, stream); break;
-    default: break;
-    }
+    const int rc = launch_format(fmt, a, tb, stream);
     if (rc || kslices == 1) return rc;
     return launch_gemm_reduce(part, kslices, (size_t)batch * w.rows, residual, y, stream);
+}
+
+int launch_regmm_gate_up(int fmt, WView gate, WView up, int cols, const _Float16 *xh,
+                         const float *rscale, int batch, float *h, void *stream)
+{
+    if (!regmm_fits(fmt, cols, batch) || gate.rows <= 0 || gate.rows % 2)
+        return (int)hipErrorInvalidValue;
+    const int tb = batch > 32 ? 2 : 1;
+    regmm::Args a{};
+    a.g.nseg = 1;
+    a.g.s[0].w = gate;
+    a.g.s[0].y = h;
+    a.g.s[0].rows = gate.rows;
+    a.g.s[0].tiles = a.rtiles = (gate.rows + 15) / 16;
+    a.up = up;
+    a.K = cols;
+    a.N = batch;
+    a.groups = 1;
+    a.kslices = 1;
+    a.xh = xh;
+    a.rscale = rscale;
+    return launch_format(fmt, a, tb, stream);
 }
 
 } // namespace hyq

@@ -339,6 +339,12 @@ template <> struct Deq<STQ1_0> {
     }
 };
 
+__device__ __forceinline__ float silu_mul(float g, float u)
+{
+    // (g / (1 + exp(-g))) * u, DenseFfn::forward (src/model.rs:680-682)
+    return (g / (1.0f + expf(-g))) * u;
+}
+
 // v_mfma 32x32 output layout: register e of a block holds row
 // 8*(e/4) + 4*(lane/32) + e%4 and column lane%32 of the block.
 __device__ __forceinline__ int acc_row_in_block(int e)

@@ -13,7 +13,8 @@ import numpy as np
 import pytest
 
 import q8_proof as P
-from synth import Q4_K, Q8_0, make_hyv3_model, make_kv_cache, load_hyv3, upload_moe
+from synth import (NAMES, Q2_0C, Q4_K, Q6_K, Q8_0, STQ1_0, make_hyv3_model, make_kv_cache,
+                   load_hyv3, upload_moe)
 
 TRACE_BYTES = 4 << 20
 
@@ -110,6 +111,26 @@ def test_moe_forward_batch(gpu_ctx, hyq, oracle, n):
     ref = oracle.moe_forward(e, H, x, n, int8_path=False)
     rel = _rel(got, ref)
     _print(f"moe batch {n} rel {rel:.2e}")
+    assert rel <= 2e-3
+
+
+@pytest.mark.parametrize("shared", [Q8_0, Q4_K, Q6_K, Q2_0C, STQ1_0], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("n", [2, 31, 33, 64, 65])
+def test_moe_shared_expert_few_tokens(gpu_ctx, hyq, oracle, shared, n):
+    """The shared expert in every format on both sides of the register-operand
+    gate/up and down (at most 64 tokens, Q6_K 32; one and two 32-token
+    blocks; a down of fewer K steps than they take at shared_mid 512)."""
+    moe = dict(MOE_C5, experts=8, used=2, mid=512, shared_mid=512 if n == 31 else 1536)
+    model = make_hyv3_model(dict(HYV3, layers=2, hidden=1024), moe, linear=Q4_K, expert=Q4_K,
+                            shared=shared, seed=5)
+    e = model["layers"][1]["moe"]
+    ffn = upload_moe(hyq, gpu_ctx, e, 1024)
+    x = np.random.default_rng(n).normal(0, 1, (n, 1024)).astype(np.float32)
+    got = ffn.forward(x)
+    ref = oracle.moe_forward(e, 1024, x, n, int8_path=False)
+    rel = _rel(got, ref)
+    _print(f"moe shared {NAMES[shared]} n {n} rel {rel:.2e}")
+    # f16 rounding of both operands of two products in a row (as above)
     assert rel <= 2e-3
 
 
