@@ -1,5 +1,5 @@
 // Batched products of few tokens with the weights dequantized straight into
-// MFMA operands (Weight::matmul at batch 2 .. regmm_max_tokens, src/quant.rs:
+// MFMA operands (Weight::matmul at batch 2 .. 64, src/quant.rs:
 // 272-344, on the f16-MFMA path): no LDS copy of either operand, no barrier
 // in the K loop.
 //
