@@ -553,10 +553,10 @@ int prefill_buffers(hyq_dense *m)
     return HYQ_OK;
 }
 
-// One chunk of n >= 2 tokens at position m->state->pos (the chunk's ids are
-// in m->pf_tok); leaves the last row's logits in m->logits and the greedy
-// token in m->token.
-int enqueue_prefill_chunk(hyq_dense *m, int n)
+// One pass of n tokens of a prompt's `total` batched ones at position
+// m->state->pos (the pass's ids are in m->pf_tok); leaves the last row's
+// logits in m->logits and the greedy token in m->token.
+int enqueue_prefill_chunk(hyq_dense *m, int n, int total)
 {
     const hyq_dense_config &c = m->cfg;
     hipStream_t st = m->ctx->stream;
@@ -613,7 +613,8 @@ int enqueue_prefill_chunk(hyq_dense *m, int n)
             // Moe::forward at batch n (src/model.rs:598-601) and the add (:602)
             HYQ_LAUNCH(launch_rms_rows(m->pf_hid, L.ffn_norm, n, H, c.rms_eps, m->pf_xn, st),
                        "rms_rows");
-            int rc = moe_ffn_rows(st, *L.moe, m->pf_xn, n, m->pf_moe, m->pf_hid, m->pf_hid);
+            int rc = moe_ffn_rows(st, *L.moe, m->pf_xn, n, total, m->pf_moe, m->pf_hid,
+                                  m->pf_hid);
             if (rc) return rc;
         } else {
         HYQ_LAUNCH(launch_norm_to_f16(m->pf_hid, n, H, L.ffn_norm, c.rms_eps, m->pf_xh,
@@ -1036,7 +1037,7 @@ int hyq_dense_prefill(hyq_dense *m, const int32_t *tokens, size_t n, float *logi
         if (s < batched) {
             HYQ_HIP(hipMemcpyAsync(m->pf_tok, tokens + s, cn * 4, hipMemcpyHostToDevice, st),
                     "hipMemcpy(tokens)");
-            if ((rc = enqueue_prefill_chunk(m, (int)cn))) return rc;
+            if ((rc = enqueue_prefill_chunk(m, (int)cn, (int)batched))) return rc;
         } else if ((rc = enqueue_step(m, true))) {
             return rc;
         }

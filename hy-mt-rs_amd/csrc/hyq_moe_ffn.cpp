@@ -202,8 +202,8 @@ MoeRowsBuf moe_rows_carve(const MoeFfn &f, int n, uint8_t *base)
     return b;
 }
 
-int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, const MoeRowsBuf &b,
-                 const float *residual, float *out)
+int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, int total,
+                 const MoeRowsBuf &b, const float *residual, float *out)
 {
     const int H = f.hidden;
     // router logits at batch n (F32, src/model.rs:691) and the pairs (:692-698)
@@ -214,15 +214,16 @@ int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, const 
     // output = shared.forward(input, n) (:699): two products, silu(g) * u, down
     HYQ_LAUNCH(launch_to_f16(xn, n, H, b.xh, b.rs, st), "to_f16");
     // (few tokens: the register-operand products, whose workgroups of 32 rows
-    // reach more CUs than the tiles of so few rows)
-    HYQ_LAUNCH(regmm_fits(f.sgate->dtype, H, n)
+    // reach more CUs than the tiles of so few rows; by the whole prompt's
+    // rows, since the two forms sum in different orders)
+    HYQ_LAUNCH(regmm_fits(f.sgate->dtype, H, total)
                    ? launch_regmm_gate_up(f.sgate->dtype, f.sgate->view, f.sup->view, H, b.xh,
                                           b.rs, n, b.h, st)
                    : launch_gate_up_f16(f.sgate->dtype, f.sgate->view, f.sup->view, H, b.xh, b.rs,
                                         n, b.h, st),
                "moe_shared_gate_up");
     HYQ_LAUNCH(launch_to_f16(b.h, n, f.smid, b.xh, b.rs, st), "to_f16");
-    HYQ_LAUNCH(regmm_fits(f.sdown->dtype, f.smid, n)
+    HYQ_LAUNCH(regmm_fits(f.sdown->dtype, f.smid, total)
                    ? launch_regmm(f.sdown->dtype, f.sdown->view, f.smid, b.xh, b.rs, n, b.ffo,
                                   nullptr, st, 1, nullptr)
                    : launch_gemm_f16(f.sdown->dtype, f.sdown->view, f.smid, b.xh, b.rs, n, b.ffo,
@@ -369,8 +370,8 @@ int hyq_moe_forward_d(hyq_ctx *ctx, const hyq_moe_config *mc, const hyq_weight *
         return moe_ffn_row(ctx->stream, f, x_d, q, moe_row_carve(f, base + off), nullptr, out_d,
                            nullptr, ctx->q8t());
     }
-    return moe_ffn_rows(ctx->stream, f, x_d, (int)tokens, moe_rows_carve(f, (int)tokens, base),
-                        nullptr, out_d);
+    return moe_ffn_rows(ctx->stream, f, x_d, (int)tokens, (int)tokens,
+                        moe_rows_carve(f, (int)tokens, base), nullptr, out_d);
 }
 
 } // extern "C"

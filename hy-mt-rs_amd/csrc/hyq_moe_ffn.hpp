@@ -66,7 +66,10 @@ size_t moe_rows_bytes(const MoeFfn &f, int n);
 MoeRowsBuf moe_rows_carve(const MoeFfn &f, int n, uint8_t *base);
 // The most rows one call takes (the grouped expert kernels' limits).
 int moe_rows_max(const MoeFfn &f);
-int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, const MoeRowsBuf &b,
-                 const float *residual, float *out);
+// n rows of a prompt that runs `total` rows in all, in passes: forms whose sums
+// run in different orders are chosen by `total`, so that a row's shared expert
+// is the same in passes of any size.
+int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, int total,
+                 const MoeRowsBuf &b, const float *residual, float *out);
 
 } // namespace hyq

@@ -42,6 +42,13 @@ int regmm_kslices(int rows, int cols)
     return ks;
 }
 
+// What the kernels take: regmm_fits, and a single row, which a pass may leave
+// over of a prompt that takes this form.
+static bool launches(int fmt, int cols, int batch)
+{
+    return batch >= 1 && regmm_fits(fmt, cols, batch < 2 ? 2 : batch);
+}
+
 static int launch_format(int fmt, const regmm::Args &a, int tb, void *stream)
 {
     switch (fmt) {
@@ -57,7 +64,7 @@ static int launch_format(int fmt, const regmm::Args &a, int tb, void *stream)
 int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rscale, int batch,
                  float *y, const float *residual, void *stream, int kslices, float *part)
 {
-    if (!regmm_fits(fmt, cols, batch) || w.rows <= 0 || kslices < 1 || (kslices > 1 && !part))
+    if (!launches(fmt, cols, batch) || w.rows <= 0 || kslices < 1 || (kslices > 1 && !part))
         return (int)hipErrorInvalidValue;
     const int tb = batch > 32 ? 2 : 1;
     regmm::Args a{};
@@ -82,7 +89,7 @@ int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rs
 int launch_regmm_gate_up(int fmt, WView gate, WView up, int cols, const _Float16 *xh,
                          const float *rscale, int batch, float *h, void *stream)
 {
-    if (!regmm_fits(fmt, cols, batch) || gate.rows <= 0 || gate.rows % 2)
+    if (!launches(fmt, cols, batch) || gate.rows <= 0 || gate.rows % 2)
         return (int)hipErrorInvalidValue;
     const int tb = batch > 32 ? 2 : 1;
     regmm::Args a{};

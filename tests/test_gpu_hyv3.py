@@ -244,6 +244,35 @@ def test_hyv3_prefill_matches_oracle(gpu_ctx, hyq, oracle):
     dec.close()
 
 
+def _prefill_bits(dec, layers, tokens, rows):
+    """Logits and every layer's appended K/V of a prompt in passes of `rows`."""
+    dec.position = 0
+    dec.set_prefill_rows(rows)
+    logits, nxt = dec.prefill(tokens)
+    kv = [a for l in range(layers) for a in dec.read_kv(l, len(tokens))]
+    return [a.view(np.uint32) for a in [logits] + kv], nxt
+
+
+@pytest.mark.parametrize("shared", [Q8_0, Q6_K], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("n,passes", [(150, (120, 64, 7)), (30, (29, 7, 1))],
+                         ids=["150_rows", "30_rows"])
+def test_moe_prefill_does_not_depend_on_the_pass_size(gpu_ctx, hyq, shared, n, passes):
+    """hyq_dense_set_prefill_rows on a model with MoE layers: the same bits for
+    a prompt of more rows than the shared expert's register-operand form takes
+    (with last passes of 30, 22 and 3 rows, which it would take) and for one
+    that it takes whole (in passes down to one row)."""
+    cfg = dict(HYV3, hidden=1024, heads=8, kv_heads=2, ffn=1024, vocab=1000)
+    moe = dict(MOE_C5, experts=8, used=2, mid=256, shared_mid=1024)
+    model = make_hyv3_model(cfg, moe, linear=Q4_K, expert=Q8_0, shared=shared, seed=6)
+    dec = load_hyv3(hyq, gpu_ctx, model, 256)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.int32)
+    one, nxt = _prefill_bits(dec, cfg["layers"], toks, 1024)
+    for rows in passes:
+        got, t = _prefill_bits(dec, cfg["layers"], toks, rows)
+        assert t == nxt and all(np.array_equal(a, b) for a, b in zip(got, one)), rows
+    dec.close()
+
+
 def test_moe_entry_point_errors(gpu_ctx, hyq):
     """The argument checks of hyq_moe_route_d / hyq_moe_forward_d (the
     reference's ensure! arms of Model::from_gguf's MoE binding,
