@@ -439,8 +439,8 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
                                        ctx->stream),
                        "f32_gemv");
         else
-            HYQ_LAUNCH(launch_f32_gemm(w->dtype, w->view, (int)w->cols, x_d, (int)batch, y_d,
-                                       ctx->stream),
+            HYQ_LAUNCH(launch_f32_gemm(w->dtype, w->view, (int)w->cols, x_d, (int)batch, (int)batch,
+                                       y_d, ctx->stream),
                        "f32_gemm");
         return HYQ_OK;
     }

@@ -332,12 +332,16 @@ int gemv_f(WView w, const WView *u, int cols, const float *x, float *y, hipStrea
 
 // The 64 x 64 tiles where they give every CU one; else 32 x 32 blocks where
 // those do, else 16 x 16 blocks (the most workgroups, the most operand reads
-// per product): each rule's line is the count below which CUs stay idle.
+// per product): each rule's line is the count below which CUs stay idle. The
+// three sum K in different orders, so the count is of `total` rows: a caller
+// that runs them in several passes gives a row the same bits in any of them.
+// Between products of different totals a row's last bits may differ (a
+// 4096-row weight: at 33 and at 193 rows).
 template <int F, bool VEC>
-int gemm_fv(WView w, int cols, const float *x, int batch, float *y, hipStream_t st)
+int gemm_fv(WView w, int cols, const float *x, int batch, int total, float *y, hipStream_t st)
 {
     auto grid = [&](int T) { return dim3((w.rows + T - 1) / T, (batch + T - 1) / T); };
-    auto count = [&](int T) { return (size_t)grid(T).x * grid(T).y; };
+    auto count = [&](int T) { return (size_t)grid(T).x * ((total + T - 1) / T); };
     if (count(64) >= 256)
         hipLaunchKernelGGL((f32_gemm_kernel<F, VEC>), grid(64), dim3(256), 0, st, w, cols, x,
                            batch, y);
@@ -351,10 +355,11 @@ int gemm_fv(WView w, int cols, const float *x, int batch, float *y, hipStream_t 
 }
 
 template <int F>
-int gemm_f(WView w, int cols, const float *x, int batch, float *y, hipStream_t st)
+int gemm_f(WView w, int cols, const float *x, int batch, int total, float *y, hipStream_t st)
 {
-    return cols % 4 == 0 && (uintptr_t)x % 16 == 0 ? gemm_fv<F, true>(w, cols, x, batch, y, st)
-                                                    : gemm_fv<F, false>(w, cols, x, batch, y, st);
+    return cols % 4 == 0 && (uintptr_t)x % 16 == 0
+               ? gemm_fv<F, true>(w, cols, x, batch, total, y, st)
+               : gemm_fv<F, false>(w, cols, x, batch, total, y, st);
 }
 
 } // namespace
@@ -370,14 +375,14 @@ int launch_f32_gemv(int fmt, WView w, const WView *up, int cols, const float *x,
     return (int)hipErrorInvalidValue;
 }
 
-int launch_f32_gemm(int fmt, WView w, int cols, const float *x, int batch, float *y,
+int launch_f32_gemm(int fmt, WView w, int cols, const float *x, int batch, int total, float *y,
                     void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     if (w.rows <= 0 || batch <= 0) return 0;
-    if (fmt == F32) return gemm_f<F32>(w, cols, x, batch, y, st);
-    if (fmt == F16) return gemm_f<F16>(w, cols, x, batch, y, st);
-    if (fmt == Q8_0) return gemm_f<Q8_0>(w, cols, x, batch, y, st);
+    if (fmt == F32) return gemm_f<F32>(w, cols, x, batch, total, y, st);
+    if (fmt == F16) return gemm_f<F16>(w, cols, x, batch, total, y, st);
+    if (fmt == Q8_0) return gemm_f<Q8_0>(w, cols, x, batch, total, y, st);
     return (int)hipErrorInvalidValue;
 }
 

@@ -273,10 +273,11 @@ bool moe_q4k_fits(int hidden, int mid);
 int moe_q4k_chunk();
 int isums_per_group(int fmt);
 // F32/F16 weights (hyq_f32mm.hip): y[rows] = W x in f32, or silu(W x) *
-// (U x) when `up` is given (batch 1); y[batch][rows] = X W^T (batch >= 1).
+// (U x) when `up` is given (batch 1); y[batch][rows] = X W^T (batch >= 1, of
+// `total` rows that a caller runs in passes).
 int launch_f32_gemv(int fmt, WView w, const WView *up, int cols, const float *x, float *y,
                     void *stream);
-int launch_f32_gemm(int fmt, WView w, int cols, const float *x, int batch, float *y,
+int launch_f32_gemm(int fmt, WView w, int cols, const float *x, int batch, int total, float *y,
                     void *stream);
 // route (hyq_route.hip): per token the `used` experts in ascending index
 // with their weights, as slot lists [tokens][used] (slot_expert,

@@ -207,7 +207,7 @@ int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, int to
 {
     const int H = f.hidden;
     // router logits at batch n (F32, src/model.rs:691) and the pairs (:692-698)
-    HYQ_LAUNCH(launch_f32_gemm(F32, f.router->view, H, xn, n, b.logits, st), "router");
+    HYQ_LAUNCH(launch_f32_gemm(F32, f.router->view, H, xn, n, total, b.logits, st), "router");
     HYQ_LAUNCH(launch_route(b.logits, f.bias_d, n, f.experts, f.used, f.normalize != 0, f.scale,
                             b.pe, b.pw, b.pt, st),
                "route");

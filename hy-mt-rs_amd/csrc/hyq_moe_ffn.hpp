@@ -67,8 +67,8 @@ MoeRowsBuf moe_rows_carve(const MoeFfn &f, int n, uint8_t *base);
 // The most rows one call takes (the grouped expert kernels' limits).
 int moe_rows_max(const MoeFfn &f);
 // n rows of a prompt that runs `total` rows in all, in passes: forms whose sums
-// run in different orders are chosen by `total`, so that a row's shared expert
-// is the same in passes of any size.
+// run in different orders are chosen by `total`, so that a row's router logits
+// and shared expert are the same in passes of any size.
 int moe_ffn_rows(hipStream_t st, const MoeFfn &f, const float *xn, int n, int total,
                  const MoeRowsBuf &b, const float *residual, float *out);
 

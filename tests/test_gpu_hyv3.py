@@ -14,7 +14,7 @@ import pytest
 
 import q8_proof as P
 from synth import (NAMES, Q2_0C, Q4_K, Q6_K, Q8_0, STQ1_0, make_hyv3_model, make_kv_cache,
-                   load_hyv3, upload_moe)
+                   load_hyv3, set_block_scale, upload_moe)
 
 TRACE_BYTES = 4 << 20
 
@@ -270,6 +270,33 @@ def test_moe_prefill_does_not_depend_on_the_pass_size(gpu_ctx, hyq, shared, n, p
     for rows in passes:
         got, t = _prefill_bits(dec, cfg["layers"], toks, rows)
         assert t == nxt and all(np.array_equal(a, b) for a, b in zip(got, one)), rows
+    dec.close()
+
+
+def test_moe_prefill_routes_alike_at_any_pass_size(gpu_ctx, hyq):
+    """A router of 1000 experts: for 240 rows its logits' product has enough
+    32 x 32 blocks to fill the GPU, for a last pass of 48 it has not, and both
+    must sum in one order: the same hidden rows after every layer (the shared
+    expert's widths keep that on one form). The bias picks the same eight
+    experts for every row, their logits ~ N(0, 16) reach where the weights
+    follow a logit's last bits, and their outputs outweigh the row they are
+    added to."""
+    cfg = dict(HYV3, hidden=256, heads=2, kv_heads=1, ffn=256, vocab=1000)
+    moe = dict(MOE_C5, experts=1000, mid=256, shared_mid=256)
+    model = make_hyv3_model(cfg, moe, linear=STQ1_0, expert=STQ1_0, shared=Q8_0, seed=8)
+    for L in model["layers"][1:]:
+        L["moe"]["router"] *= 4
+        L["moe"]["bias"][:8] = 5
+        set_block_scale(STQ1_0, L["moe"]["gate"], 0.2)
+        set_block_scale(STQ1_0, L["moe"]["down"], 8.0)
+    dec = load_hyv3(hyq, gpu_ctx, model, 256)
+    toks = np.random.default_rng(8).integers(0, cfg["vocab"], 240).astype(np.int32)
+    dec.set_trace(240)
+    one, nxt = _prefill_bits(dec, cfg["layers"], toks, 1024)
+    whole = dec.trace(240)[:, -48:].view(np.uint32)
+    got, t = _prefill_bits(dec, cfg["layers"], toks, 64)
+    assert np.array_equal(dec.trace(48).view(np.uint32), whole)
+    assert t == nxt and all(np.array_equal(a, b) for a, b in zip(got, one))
     dec.close()
 
 
