@@ -423,122 +423,9 @@ __global__ __launch_bounds__(256) void moe_plan_kernel(const int *__restrict__ p
     for (int q = t; q < nv; q += 256) tlist[toff[tkey(q)] + rank[q]] = q;
 }
 
-// The plan for up to PLAN_SMALL pairs (and at most PLAN_SMALL tokens and
-// experts) with every intermediate in LDS: the same outputs as
-// moe_plan_kernel, without its global round trips between the steps.
-constexpr int PLAN_SMALL = 2048;
-
-__device__ void lds_exclusive_scan(const int *cnt, int n, int *off, int *lsum)
-{
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int per = (n + 255) / 256;
-    const int lo = t * per, hi = min(n, lo + per);
-    int s = 0;
-    for (int i = lo; i < hi; ++i) s += cnt[i];
-    int v = s;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int u = __shfl_up(v, d);
-        if (lane >= d) v += u;
-    }
-    if (lane == 63) lsum[w] = v;
-    __syncthreads();
-    int wb = 0;
-    for (int j = 0; j < w; ++j) wb += lsum[j];
-    int run = wb + v - s;
-    for (int i = lo; i < hi; ++i) {
-        off[i] = run;
-        run += cnt[i];
-    }
-    if (t == 255) off[n] = wb + v;
-    __syncthreads();
-}
-
-// rank[i] = number of j < i with key[j] == key[i] (key < 0 skipped), cnt[k]
-// = count of key k; all arrays in LDS, key 16-byte aligned and padded with
-// -1 to a multiple of 4.
-__device__ void lds_stable_rank(const int *key, int n, int *cnt, int nkeys, int *rank)
-{
-    const int t = threadIdx.x;
-    for (int k = t; k < nkeys; k += 256) cnt[k] = 0;
-    __syncthreads();
-    for (int base = 0; base < n; base += 256) {
-        const int i = base + t;
-        const int k = i < n ? key[i] : -1;
-        if (k >= 0) {
-            const int4 *l4 = reinterpret_cast<const int4 *>(key + base);
-            int r = 0;
-#pragma unroll 4
-            for (int j = 0; j < (t >> 2); ++j) {
-                const int4 v = l4[j];
-                r += (v.x == k) + (v.y == k) + (v.z == k) + (v.w == k);
-            }
-            for (int j = t & ~3; j < t; ++j) r += key[base + j] == k;
-            rank[i] = cnt[k] + r;
-        }
-        __syncthreads();
-        if (k >= 0) atomicAdd(&cnt[k], 1);
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(256) void moe_plan_small_kernel(
-    const int *__restrict__ ptok, const int *__restrict__ pexp, int P, int T, int E, int *eoff,
-    int *order, int *toff, int *tlist, int *tiles, int *ntiles, int chunk)
-{
-    __shared__ int cnt[PLAN_SMALL];
-    __shared__ int off[PLAN_SMALL + 1];
-    __shared__ __attribute__((aligned(16))) int key[PLAN_SMALL + 4];
-    __shared__ int tok[PLAN_SMALL];
-    __shared__ int ord[PLAN_SMALL];
-    __shared__ int rank[PLAN_SMALL + 1];
-    __shared__ int lsum[4];
-    const int t = threadIdx.x;
-    const int P4 = (P + 3) & ~3;
-    for (int p = t; p < P4; p += 256) {
-        int e = -1, tk = -1;
-        if (p < P) {
-            tk = ptok[p];
-            e = pexp[p];
-            if (!(tk >= 0 && tk < T && e >= 0 && e < E)) e = -1;
-        }
-        key[p] = e;
-        tok[p] = tk;
-    }
-    __syncthreads();
-    // group pairs by expert (stable)
-    lds_stable_rank(key, P, cnt, E, rank);
-    lds_exclusive_scan(cnt, E, off, lsum);
-    for (int e = t; e <= E; e += 256) eoff[e] = off[e];
-    for (int p = t; p < P; p += 256)
-        if (key[p] >= 0) ord[off[key[p]] + rank[p]] = p;
-    __syncthreads();
-    const int nv = off[E];
-    for (int q = t; q < nv; q += 256) order[q] = ord[q];
-    // chunk-token chunks of every expert
-    for (int e = t; e < E; e += 256) cnt[e] = (off[e + 1] - off[e] + chunk - 1) / chunk;
-    __syncthreads();
-    lds_exclusive_scan(cnt, E, rank, lsum); // rank[0..E]: chunk offsets
-    for (int e = t; e < E; e += 256)
-        for (int c = 0; c < cnt[e]; ++c) {
-            tiles[2 * (rank[e] + c)] = e;
-            tiles[2 * (rank[e] + c) + 1] = c;
-        }
-    if (t == 0) *ntiles = rank[E];
-    __syncthreads();
-    // for each token, its positions in ascending expert order
-    const int nv4 = (nv + 3) & ~3;
-    for (int q = t; q < nv4; q += 256) key[q] = q < nv ? tok[ord[q]] : -1;
-    __syncthreads();
-    lds_stable_rank(key, nv, cnt, T, rank);
-    lds_exclusive_scan(cnt, T, off, lsum);
-    for (int k = t; k <= T; k += 256) toff[k] = off[k];
-    for (int q = t; q < nv; q += 256) tlist[off[key[q]] + rank[q]] = q;
-}
-
 // The plan for up to PLAN_FAST pairs, tokens and experts, with at most
 // PLAN_FAST_TAB (batch, key) cells per grouping, on 1024 threads: the same
-// outputs as moe_plan_small_kernel. A grouping's stable rank comes from
+// outputs as moe_plan_kernel. A grouping's stable rank comes from
 // bit masks instead of pairwise compares: in batch b (64 consecutive
 // elements, one wave) every lane sets its bit in the mask of (b, its key)
 // with one LDS atomic OR, so the bits below its own give its rank among the
@@ -1318,10 +1205,6 @@ int launch_moe(int fmt_gu, int fmt_down, WView gate, WView up, WView down, int h
                            ctok, xf);
     else if (plan_mid_fits(npairs, tokens, experts))
         hipLaunchKernelGGL(moe_plan_mid_kernel, dim3(2), dim3(1024), 0, st, ptok, pexp, npairs,
-                           tokens, experts, eoff, order, toff, tlist, tiles, ntiles,
-                           few ? moe_q4k_chunk() : BN);
-    else if (npairs <= PLAN_SMALL && tokens <= PLAN_SMALL && experts <= PLAN_SMALL)
-        hipLaunchKernelGGL(moe_plan_small_kernel, dim3(1), dim3(256), 0, st, ptok, pexp, npairs,
                            tokens, experts, eoff, order, toff, tlist, tiles, ntiles,
                            few ? moe_q4k_chunk() : BN);
     else

@@ -232,11 +232,14 @@ def test_moe_row_group_streams(gpu_ctx, hyq, oracle, hidden, mid):
 
 
 @pytest.mark.parametrize("tokens,experts,used", [(300, 64, 8), (1024, 64, 8), (4096, 5, 2),
-                                                 (700, 200, 5), (129, 1000, 8)])
+                                                 (700, 200, 5), (129, 1000, 8), (2000, 16, 8),
+                                                 (1000, 700, 8), (200, 1500, 8)])
 def test_moe_plan_of_many_pairs(gpu_ctx, hyq, oracle, tokens, experts, used):
     """More pairs than the 1024-pair plan takes, in a random order, with
     pairs out of range (skipped) and a token routed nowhere: sampled tokens
-    against the f64 chain, and the same call twice (one scratch) bit for bit."""
+    against the f64 chain, and the same call twice (one scratch) bit for bit.
+    The last three are past the plan in LDS: by the pairs (15992), by its
+    (batch, expert) cells (125 x 700) and by the experts."""
     hidden, mid = 256, 256
     gate = random_matrix(Q4_K, experts * mid, hidden, seed=41)
     up = random_matrix(Q4_K, experts * mid, hidden, seed=42)
