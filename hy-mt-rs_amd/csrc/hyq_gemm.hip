@@ -616,7 +616,9 @@ __global__ __launch_bounds__(1024) void moe_plan_fast_kernel(
 // the count in tab[key][batch], and each key's exclusive scan over the batches
 // runs across a wave's lanes. A token's positions are collected in any order
 // (LDS atomics) and then placed by counting the smaller ones of the same
-// token, a list as long as the experts a token uses.
+// token, a list as long as the experts a token uses; one of more than PLAN_LONG
+// pairs (a caller may repeat an expert) sets its positions in a bit map and
+// counts the bits below (8190 pairs of one token: 3.2 ms by the list, 29 us so).
 // Bound: one workgroup's chain of LDS passes. 4000 pairs of 64 experts:
 // moe_plan_kernel (256 threads, pairwise compares, the intermediates in
 // global memory) 134.7 us, this 11.8 us.
@@ -624,6 +626,8 @@ constexpr int PLAN_MID = 8192;
 constexpr int PLAN_MID_EXPERTS = 1024;
 constexpr int PLAN_MID_CELLS = 32768;
 constexpr int PLAN_MID_PER = PLAN_MID / 1024; // pairs per thread
+constexpr int PLAN_LONG = 256;
+constexpr int PLAN_LONGS = PLAN_MID / PLAN_LONG; // tokens of more pairs than that
 
 __host__ __device__ inline bool plan_mid_fits(int P, int T, int E)
 {
@@ -635,11 +639,12 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
     const int *__restrict__ ptok, const int *__restrict__ pexp, int P, int T, int E, int *eoff,
     int *order, int *toff, int *tlist, int *tiles, int *ntiles, int chunk)
 {
-    __shared__ uint16_t tab[PLAN_MID_CELLS]; // [key][batch]
+    __shared__ __align__(4) uint16_t tab[PLAN_MID_CELLS]; // [key][batch]
     __shared__ int off[PLAN_MID_EXPERTS + 1];
     __shared__ int lsum[16];
     __shared__ int cnt[PLAN_MAX + 1];   // workgroup 0: tile offsets, 1: token offsets
     __shared__ uint16_t list[PLAN_MID]; // workgroup 1: positions by token
+    __shared__ int longs[PLAN_LONGS], nlongs;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int nb = (P + 63) / 64;
     const bool tokens_wg = blockIdx.x == 1;
@@ -657,6 +662,7 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
     for (int i = t; i < nb * E; i += 1024) tab[i] = 0;
     if (tokens_wg)
         for (int i = t; i <= T; i += 1024) cnt[i] = 0;
+    if (t == 0) nlongs = 0;
     __syncthreads();
     const int bits = 32 - __clz(E);
     const unsigned long long below = (1ull << lane) - 1;
@@ -730,13 +736,58 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
 #pragma unroll
     for (int j = 0; j < PLAN_MID_PER; ++j)
         if (pos[j] >= 0) list[cnt[tok[j]] + slot[j]] = (uint16_t)pos[j];
+    // (tab is free: every count in it was read before the scan's barriers)
+    unsigned *map = reinterpret_cast<unsigned *>(tab); // [PLAN_LONGS][PLAN_MID / 32]
+    constexpr int WORDS = PLAN_MID / 32;
+    for (int k = t; k < T; k += 1024)
+        if (cnt[k + 1] - cnt[k] > PLAN_LONG) longs[atomicAdd(&nlongs, 1)] = k;
+    for (int i = t; i < PLAN_LONGS * WORDS; i += 1024) map[i] = 0;
     __syncthreads();
+    const int nl = nlongs;
+    // the row of bits of the pair's token; -1 for a short list
+    auto long_row = [&](int j) {
+        int r = -1;
+        for (int i = 0; i < nl; ++i)
+            if (longs[i] == tok[j]) r = i;
+        return r;
+    };
+    if (nl) { // (the workgroup's test)
+#pragma unroll
+        for (int j = 0; j < PLAN_MID_PER; ++j) {
+            const int r = pos[j] >= 0 ? long_row(j) : -1;
+            if (r >= 0) atomicOr(&map[r * WORDS + (pos[j] >> 5)], 1u << (pos[j] & 31));
+        }
+        __syncthreads();
+        // bits before each word, over the lists (no longer needed for these tokens)
+        for (int r = w; r < nl; r += 16) {
+            const int lo = cnt[longs[r]];
+            int carry = 0;
+            for (int i0 = 0; i0 < WORDS; i0 += 64) {
+                const int c = __popc(map[r * WORDS + i0 + lane]);
+                int x = c;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const int u = __shfl_up(x, d);
+                    if (lane >= d) x += u;
+                }
+                list[lo + i0 + lane] = (uint16_t)(carry + x - c);
+                carry += wave::lane(x, 63);
+            }
+        }
+        __syncthreads();
+    }
 #pragma unroll
     for (int j = 0; j < PLAN_MID_PER; ++j)
         if (pos[j] >= 0) {
             const int lo = cnt[tok[j]], hi = cnt[tok[j] + 1];
             int r = lo;
-            for (int i = lo; i < hi; ++i) r += list[i] < pos[j];
+            if (hi - lo > PLAN_LONG) {
+                const int word = pos[j] >> 5;
+                r += list[lo + word] + __popc(map[long_row(j) * WORDS + word] &
+                                              ((1u << (pos[j] & 31)) - 1u));
+            } else {
+                for (int i = lo; i < hi; ++i) r += list[i] < pos[j];
+            }
             tlist[r] = pos[j];
         }
 }

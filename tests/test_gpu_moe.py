@@ -284,6 +284,42 @@ def test_moe_plan_of_many_pairs(gpu_ctx, hyq, oracle, tokens, experts, used):
         w.release()
 
 
+@pytest.mark.parametrize("counts", [(8190,), (257, 3000, 256, 258, 1, 300), (256,) * 31 + (200,),
+                                    (263,) * 31 + (30,)],
+                         ids=["one_token", "around_the_limit", "31_at_256", "31_above"])
+def test_moe_plan_of_repeated_experts(gpu_ctx, hyq, oracle, counts):
+    """Tokens of more than 256 pairs, which repeat experts (the pair list may):
+    their order in the routed sum comes from a bit map, the same positions as
+    by counting. Experts whose outputs differ by powers of two make a sum in
+    another order show, and the call of more pairs than that plan takes (the
+    pairs and their weights of 0 to one more token) gives the same bits."""
+    hidden, mid, experts, tokens = 256, 256, 16, len(counts) + 1
+    w = [random_matrix(Q4_K, experts * r, c, seed=71 + i) for i, (r, c) in
+         enumerate(((mid, hidden), (mid, hidden), (hidden, mid)))]
+    rng = np.random.default_rng(sum(counts))
+    pt = np.repeat(np.arange(len(counts), dtype=np.int32), counts)
+    pe = rng.integers(0, experts, pt.size).astype(np.int32)
+    pw = (rng.uniform(0.1, 1.0, pt.size) * 2.0 ** -rng.integers(0, 12, pt.size)).astype(np.float32)
+    perm = rng.permutation(pt.size)
+    pt, pe, pw = pt[perm], pe[perm], pw[perm]
+    x = rng.normal(0, 1, tokens * hidden).astype(np.float32)
+    W = [gpu_ctx.upload(Q4_K, a, d) for a, d in zip(w, ((hidden, mid, experts),) * 2
+                                                    + ((mid, hidden, experts),))]
+    zero = np.zeros(tokens * hidden, np.float32)
+    got = hyq.moe_experts(*W, x, tokens, pt, pe, pw, zero).reshape(tokens, hidden)
+    more = 8193 - pt.size
+    want = hyq.moe_experts(*W, x, tokens, np.concatenate([pt, np.full(more, tokens - 1, np.int32)]),
+                           np.concatenate([pe, np.zeros(more, np.int32)]),
+                           np.concatenate([pw, np.zeros(more, np.float32)]),
+                           zero).reshape(tokens, hidden)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    ref, mag = chain_f64(oracle, Q4_K, Q4_K, *w, hidden, mid, x, pt, pe, pw,
+                         zero.reshape(tokens, hidden), [0])
+    check_moe(got[0], ref[0], mag[0], "token 0")
+    for a in W:
+        a.release()
+
+
 def test_moe_device_entry_point_and_rerun(gpu_ctx, hyq):
     """hyq_moe_experts_d on device buffers equals the host entry point, twice
     in a row on the same scratch (the second with fewer pairs)."""
