@@ -332,20 +332,27 @@ int gemv_f(WView w, const WView *u, int cols, const float *x, float *y, hipStrea
 
 // The 64 x 64 tiles where they give every CU one; else 32 x 32 blocks where
 // those do, else 16 x 16 blocks (the most workgroups, the most operand reads
-// per product): each rule's line is the count below which CUs stay idle. The
-// three sum K in different orders, so the count is of `total` rows: a caller
+// per product): each rule's line is the count below which CUs stay idle. Below
+// 512 columns a 16 x 16 block's sixteen waves have too little to split and a CU
+// holds one block, so 32 x 32 blocks take those ([300 x 96] F32: 777 rows 15.8
+// -> 3.9 us, 64 rows 5.0 -> 3.8; [64 x 252] 64 rows 6.8 -> 3.6), with
+// single-value loads, which favour more waves, from 256 columns only past one
+// round of 16 x 16 blocks ([64 x 257] 64 rows 6.0 against 7.5; [300 x 257] 250
+// rows 10.7 -> 8.0).
+// The three sum K in different orders, so the count is of `total` rows: a caller
 // that runs them in several passes gives a row the same bits in any of them.
-// Between products of different totals a row's last bits may differ (a
-// 4096-row weight: at 33 and at 193 rows).
+// Between products of different totals a row's last bits may differ ([4096 x
+// 4096]: at 33 and at 193 rows).
 template <int F, bool VEC>
 int gemm_fv(WView w, int cols, const float *x, int batch, int total, float *y, hipStream_t st)
 {
     auto grid = [&](int T) { return dim3((w.rows + T - 1) / T, (batch + T - 1) / T); };
     auto count = [&](int T) { return (size_t)grid(T).x * ((total + T - 1) / T); };
+    const bool narrow = cols < 512 && (VEC || cols < 256 || count(16) > 256);
     if (count(64) >= 256)
         hipLaunchKernelGGL((f32_gemm_kernel<F, VEC>), grid(64), dim3(256), 0, st, w, cols, x,
                            batch, y);
-    else if (count(32) >= 256)
+    else if (narrow || count(32) >= 256)
         hipLaunchKernelGGL((f32_gemm_split_kernel<F, VEC, 32>), grid(32), dim3(64 * split_waves(32)),
                            0, st, w, cols, x, batch, y);
     else

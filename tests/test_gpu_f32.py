@@ -70,14 +70,17 @@ def test_qkv_and_gate_up_of_decoded_rows(gpu_ctx, oracle, dtype):
 
 
 # The batched product's three forms (16 x 16 and 32 x 32 blocks with K split
-# over eight waves, 64 x 64 tiles) at ragged rows, batches and widths, and
-# widths or an input address that only single-value loads can read. The bound
+# over sixteen and eight waves, 64 x 64 tiles) at ragged rows, batches and
+# widths, on both sides of the lines between them, and widths or an input
+# address that only single-value loads can read. The bound
 # is the file's: a sum of K f32 terms in any order errs by at most
 # K * 2^-24 * sum|w x|, far below 1e-5 * sum|w x| for these K.
 @pytest.mark.parametrize("dtype,rows,cols,batch,shift", [
     (F32, 64, 2048, 500, 0), (F16, 17, 129, 33, 0), (F32, 5, 4, 2, 0), (F32, 64, 2048, 64, 1),
     (F32, 1000, 257, 300, 0), (F16, 1000, 260, 290, 0), (Q8_0, 1100, 96, 257, 0),
-    (F32, 1500, 33, 700, 0), (F16, 1025, 1036, 1000, 0), (F16, 1025, 64, 1000, 1)])
+    (F32, 1500, 33, 700, 0), (F16, 1025, 1036, 1000, 0), (F16, 1025, 64, 1000, 1),
+    (F16, 17, 513, 33, 0), (F32, 5, 516, 2, 0), (F32, 70, 508, 65, 0), (F16, 256, 257, 256, 0),
+    (F32, 257, 257, 256, 1), (Q8_0, 40, 544, 31, 0)])
 def test_batched_forms_at_their_edges(gpu_ctx, hyq, oracle, dtype, rows, cols, batch, shift):
     w = random_matrix(dtype, rows, cols, seed=rows + cols)
     x = np.random.default_rng(batch).normal(0, 1, batch * cols).astype(np.float32)
@@ -94,11 +97,11 @@ def test_batched_forms_at_their_edges(gpu_ctx, hyq, oracle, dtype, rows, cols, b
     W.release()
 
 
-@pytest.mark.parametrize("rows,batch", [(64, 40), (1000, 300), (1500, 700)])
-def test_batched_products_keep_small_and_non_finite_values(gpu_ctx, rows, batch):
+@pytest.mark.parametrize("rows,batch,cols", [(64, 40, 96), (1000, 300, 96), (1500, 700, 96),
+                                             (64, 40, 528)])
+def test_batched_products_keep_small_and_non_finite_values(gpu_ctx, rows, batch, cols):
     """A column of subnormal weights, an infinity and a NaN in single rows:
     each only reaches its own outputs."""
-    cols = 96
     w = np.random.default_rng(1).normal(0, 1, (rows, cols)).astype(np.float32)
     w[1] = 0
     w[1, 5] = 1e-39

@@ -274,14 +274,13 @@ def test_moe_prefill_does_not_depend_on_the_pass_size(gpu_ctx, hyq, shared, n, p
 
 
 def test_moe_prefill_routes_alike_at_any_pass_size(gpu_ctx, hyq):
-    """A router of 1000 experts: for 240 rows its logits' product has enough
-    32 x 32 blocks to fill the GPU, for a last pass of 48 it has not, and both
-    must sum in one order: the same hidden rows after every layer (the shared
-    expert's widths keep that on one form). The bias picks the same eight
+    """A router of 1000 experts: for 240 rows its logits' product takes 32 x 32
+    blocks, a product of 48 rows (the last pass) would take 16 x 16 ones, and
+    both must sum in one order: the same hidden rows after every layer. The bias picks the same eight
     experts for every row, their logits ~ N(0, 16) reach where the weights
     follow a logit's last bits, and their outputs outweigh the row they are
     added to."""
-    cfg = dict(HYV3, hidden=256, heads=2, kv_heads=1, ffn=256, vocab=1000)
+    cfg = dict(HYV3, hidden=512, heads=2, kv_heads=1, ffn=256, vocab=1000)
     moe = dict(MOE_C5, experts=1000, mid=256, shared_mid=256)
     model = make_hyv3_model(cfg, moe, linear=STQ1_0, expert=STQ1_0, shared=Q8_0, seed=8)
     for L in model["layers"][1:]:
