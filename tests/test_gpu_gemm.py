@@ -8,6 +8,7 @@ term's relative error by 2*2^-11 < 1e-3) and 2e-3 relative in the 2-norm."""
 import numpy as np
 import pytest
 
+import tile_cases
 from gpu_util import check_prefill_path
 from synth import NAMES, Q2_0C, Q4_K, Q6_K, Q8_0, QUANT, STQ1_0, random_matrix, row_bytes
 
@@ -67,11 +68,10 @@ def test_prefill_7b_full_size_sampled_rows(gpu_ctx, oracle, dtype, rows, cols):
                                                    (Q4_K, 6144, 4096, 257), (Q4_K, 6112, 4096, 300)],
                          ids=["gate_up_q4k_300", "down_q6k_270", "qkv_q4k_257", "rows96_partial_300"])
 def test_prefill_7b_ragged_token_blocks(gpu_ctx, oracle, dtype, rows, cols, batch):
-    """The 256-token tiles with their activations in fragment order at token
-    counts that end inside a 32-token block (and inside a 256-token tile):
-    sampled weight rows, all tokens, against the oracle; the partial block's
-    rows past the batch feed sums that are never written. [6144 x 4096] and
-    [6112 x 4096] run as 96-row tiles (the latter's last tile 64 rows)."""
+    """7B shapes at token counts that end inside a 32-token block (and inside
+    a tile), their activations in fragment order: sampled weight rows, all
+    tokens, against the oracle; the partial block's rows past the batch feed
+    sums that are never written."""
     _print("gemm ragged", NAMES[dtype], rows, cols, batch)
     w = random_matrix(dtype, rows, cols, seed=rows + batch)
     x = np.random.default_rng(batch).normal(0, 1, batch * cols).astype(np.float32)
@@ -86,11 +86,10 @@ def test_prefill_7b_ragged_token_blocks(gpu_ctx, oracle, dtype, rows, cols, batc
 
 
 def test_fragment_tiles_equal_row_tiles(gpu_ctx):
-    """At 300 tokens a [14336 x 4096] product runs as 256-token tiles with its
-    activations in fragment order; at 200 tokens the same weight runs as
-    128-token tiles with its activations copied through LDS. The same
-    operands meet in the same k order either way, so the first 200 token rows
-    agree bit for bit."""
+    """A [14336 x 4096] product runs as tiles of 128 rows x 192 tokens at 300
+    tokens and of 64 rows x 256 tokens at 200. The same operands meet in the
+    same k order either way, so the first 200 token rows agree bit for
+    bit."""
     rows, cols = 14336, 4096
     w = random_matrix(Q4_K, rows, cols, seed=11)
     x = np.random.default_rng(11).normal(0, 1, 300 * cols).astype(np.float32)
@@ -258,12 +257,36 @@ def test_register_operand_products(gpu_ctx, hyq, oracle, dtype, rows, cols):
 
 
 @pytest.mark.parametrize("dtype", QUANT, ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("shape,rows,batch", tile_cases.MATMUL)
+def test_tile_shapes(gpu_ctx, oracle, dtype, shape, rows, batch):
+    """Every tile shape in every format with partial row and token tiles (which
+    product takes which shape: tests/tile_cases.py): all tokens of sampled weight
+    rows, the first ones and the last row tile among them, against the
+    oracle."""
+    cols = 512 if dtype == Q2_0C else 256
+    _print("tile", shape, NAMES[dtype], rows, batch)
+    w = random_matrix(dtype, rows, cols, seed=rows + dtype)
+    x = np.random.default_rng(batch).normal(0, 1, batch * cols).astype(np.float32)
+    W = gpu_ctx.upload(dtype, w, (cols, rows))
+    y = W.matmul(x, batch).reshape(batch, rows)
+    assert np.all(np.isfinite(y))
+    pick = np.unique(np.concatenate([np.arange(8), np.arange(rows - 100, rows),
+                                     np.random.default_rng(rows).choice(rows, 60)]))
+    sub = w.reshape(rows, -1)[pick].reshape(-1)
+    y_ref, mag = oracle.matmul_f64(dtype, sub, len(pick), cols, x, batch)
+    check_prefill_path(y[:, pick], y_ref.reshape(batch, -1), mag.reshape(batch, -1),
+                       f"{shape} {NAMES[dtype]}")
+    W.release()
+
+
+@pytest.mark.parametrize("dtype", QUANT, ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("rows,cols", [(200, 1024), (130, 2560)], ids=["200x1024", "130x2560"])
 def test_tile_shapes_at_block_edges(gpu_ctx, oracle, dtype, rows, cols):
-    """Token counts on both sides of every tile shape (128, 192 and 256 tokens)
-    and of a wave's token blocks, rows that end inside a tile: parity with the
-    oracle, which is token-local; on one side of 128 tokens (the K split's
-    classes) a token's row has the same bits at any count."""
+    """Token counts on both sides of every tile's (128, 192 and 256 tokens) and
+    of a wave's token blocks, rows that end inside a tile, in the shape that few
+    row tiles take (64 rows x 256 tokens): parity with the oracle, which is
+    token-local; on one side of 128 tokens (the K split's classes) a token's
+    row has the same bits at any count."""
     _print("tile shapes", NAMES[dtype], rows, cols)
     w = random_matrix(dtype, rows, cols, seed=rows + dtype)
     top = 520

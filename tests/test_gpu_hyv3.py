@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import q8_proof as P
+import tile_cases
 from synth import (NAMES, Q2_0C, Q4_K, Q6_K, Q8_0, STQ1_0, make_hyv3_model, make_kv_cache,
                    load_hyv3, set_block_scale, upload_moe)
 
@@ -131,6 +132,33 @@ def test_moe_shared_expert_few_tokens(gpu_ctx, hyq, oracle, shared, n):
     rel = _rel(got, ref)
     _print(f"moe shared {NAMES[shared]} n {n} rel {rel:.2e}")
     # f16 rounding of both operands of two products in a row (as above)
+    assert rel <= 2e-3
+
+
+@pytest.mark.parametrize("shared", [Q8_0, Q4_K, Q6_K, Q2_0C, STQ1_0], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("shape,smid,n", tile_cases.GATE_UP)
+def test_gate_up_tile_shapes(gpu_ctx, hyq, oracle, shared, shape, smid, n):
+    """The gate/up product in every tile shape (tests/tile_cases.py) and format
+    with a partial token tile, as the shared expert of a small MoE FFN: sampled
+    rows, the last token tile's among them, at the file's bar of a batch, 2e-3 of
+    the sample's norm: f16 roundings of 2^-11 of both operands of two products
+    in a row. (Per row there is no such bound: Q4_K weights have a mean, so
+    a row whose values nearly sum to zero has small products of large terms.)
+    Four gate rows left out in one sampled row would be 5e-3. The experts'
+    outputs are small beside it (STQ1_0 blocks of scale ~ 0.02)."""
+    H = 512
+    moe = dict(MOE_C5, experts=2, used=1, mid=256, shared_mid=smid)
+    model = make_hyv3_model(dict(HYV3, layers=2, hidden=H, ffn=512, vocab=256), moe, linear=Q4_K,
+                            expert=STQ1_0, shared=shared, seed=9)
+    e = model["layers"][1]["moe"]
+    ffn = upload_moe(hyq, gpu_ctx, e, H)
+    x = np.random.default_rng(n).normal(0, 1, (n, H)).astype(np.float32)
+    got = ffn.forward(x)
+    pick = np.unique(np.concatenate([[0, 31, 32, 127, 128, 191, 192, 255, n - 33, n - 1],
+                                     np.random.default_rng(smid).choice(n, 14)]))
+    ref = oracle.moe_forward(e, H, x[pick], len(pick), int8_path=False)
+    rel = _rel(got[pick], ref)
+    _print(f"gate/up {shape} {NAMES[shared]} rel {rel:.2e}")
     assert rel <= 2e-3
 
 
