@@ -68,15 +68,13 @@ int launch_regmm(int fmt, WView w, int cols, const _Float16 *xh, const float *rs
         return (int)hipErrorInvalidValue;
     const int tb = batch > 32 ? 2 : 1;
     regmm::Args a{};
-    a.g.nseg = 1;
-    a.g.s[0].w = w;
-    a.g.s[0].y = y;
-    a.g.s[0].residual = residual;
-    a.g.s[0].rows = w.rows;
-    a.g.s[0].tiles = a.rtiles = (w.rows + 31) / 32;
+    a.w = w;
+    a.y = y;
+    a.residual = residual;
+    a.rows = w.rows;
+    a.rtiles = (w.rows + 31) / 32;
     a.K = cols;
     a.N = batch;
-    a.groups = (batch + 32 * tb - 1) / (32 * tb);
     a.kslices = kslices;
     a.xh = xh;
     a.rscale = rscale;
@@ -93,15 +91,13 @@ int launch_regmm_gate_up(int fmt, WView gate, WView up, int cols, const _Float16
         return (int)hipErrorInvalidValue;
     const int tb = batch > 32 ? 2 : 1;
     regmm::Args a{};
-    a.g.nseg = 1;
-    a.g.s[0].w = gate;
-    a.g.s[0].y = h;
-    a.g.s[0].rows = gate.rows;
-    a.g.s[0].tiles = a.rtiles = (gate.rows + 15) / 16;
+    a.w = gate;
     a.up = up;
+    a.y = h;
+    a.rows = gate.rows;
+    a.rtiles = (gate.rows + 15) / 16;
     a.K = cols;
     a.N = batch;
-    a.groups = 1;
     a.kslices = 1;
     a.xh = xh;
     a.rscale = rscale;

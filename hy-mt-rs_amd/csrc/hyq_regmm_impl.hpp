@@ -14,9 +14,9 @@
 // Measured, with the f16 rows' launch (LDS engine -> this): Q2_0C
 // [6144 x 2048] 21 tokens 17.0 -> 10.1 us, 64 tokens 22.4 -> 12.1; Q4_K
 // [14336 x 4096] 21 tokens 44.5 -> 23.4, 64 tokens 48.5 -> 28.4; Q6_K
-// [4096 x 14336] 21 tokens 46.5 -> 36.1.
+// [4096 x 4096] 20 tokens 14.2 (where it stays with the engine: hyq_regmm.hip).
 //
-// Form. A workgroup owns 32 weight rows against TB blocks of 32 tokens; its
+// Form. A workgroup owns 32 weight rows against the TB blocks of 32 tokens; its
 // waves split K in 64-column steps, each wave with all of the workgroup's rows
 // and tokens, and meet once, in LDS, where the waves' sums are added in wave
 // order. Lane l of a wave is weight row l % 32 and
@@ -73,12 +73,13 @@ template <int F, int TB> constexpr int occupancy()
 }
 
 struct Args {
-    GemmSegs g; // .tiles: row tiles of 32 rows
-    int K, N, groups, rtiles, kslices;
-    const _Float16 *xh; // fragment order
+    WView w, up; // up: GU, w is gate
+    float *y;
+    const float *residual;
+    int rows, rtiles, K, N, kslices; // rtiles: of 32 rows (GU: 16 of each)
+    const _Float16 *xh;              // fragment order
     const float *rscale;
     float *part; // [kslices][N][rows] when kslices > 1
-    WView up;    // GU: segment 0 is gate
 };
 
 template <int F, int TB, bool GU>
@@ -86,15 +87,11 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
 {
     using D = Deq<F>;
     __shared__ float4 red[TB][WAVES][4][64];
-    const int total = a.rtiles * a.groups, per = (total + 7) / 8;
+    const int per = (a.rtiles + 7) / 8;
     const int T = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8); // XCD-contiguous
-    if (T >= total || (int)(blockIdx.x / 8) >= per) return;
-    int rt = T / a.groups, sg = 0;
-    const int n0 = (T % a.groups) * (32 * TB);
-    while (sg + 1 < a.g.nseg && rt >= a.g.s[sg].tiles) rt -= a.g.s[sg++].tiles;
-    const GemmSeg &S = a.g.s[sg];
-    const int M = S.rows, K = a.K, N = a.N;
-    const int m0 = rt * (GU ? 16 : 32);
+    if (T >= a.rtiles) return;
+    const int M = a.rows, K = a.K, N = a.N;
+    const int m0 = T * (GU ? 16 : 32);
     const int t = threadIdx.x, lane = t & 63, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
 
@@ -114,8 +111,8 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
     if (c0 < c1) {
         // (rows past the end: unused)
         const int q = lane & 31;
-        const RowPtr rp = GU ? D::rows(q & 2 ? a.up : S.w, min(m0 + 2 * (q >> 2) + (q & 1), M - 1))
-                             : D::rows(S.w, min(m0 + q, M - 1));
+        const RowPtr rp = GU ? D::rows(q & 2 ? a.up : a.w, min(m0 + 2 * (q >> 2) + (q & 1), M - 1))
+                             : D::rows(a.w, min(m0 + q, M - 1));
         const _Float16 *xb[TB];
         const int nblk = (N + 31) / 32;
         // piece(i, h) = piece(i, 0) + h * (piece(0, 1) - piece(0, 0))
@@ -123,7 +120,7 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
         unsigned pstride[TB]; // halves per piece of the block
 #pragma unroll
         for (int b = 0; b < TB; ++b) {
-            const int blk = min(n0 / 32 + b, nblk - 1), c = min(32, N - 32 * blk);
+            const int blk = min(b, nblk - 1), c = min(32, N - 32 * blk);
             pstride[b] = 8 * c;
             xb[b] = a.xh + (size_t)blk * 32 * K + min(lane & 31, c - 1) * 8 + hoff * 8 * c;
         }
@@ -184,7 +181,7 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
     if (m >= M) return;
 #pragma unroll
     for (int b = 0; b < TB; ++b) {
-        const int n = n0 + 32 * b + (lane & 31);
+        const int n = 32 * b + (lane & 31);
         if (n >= N) continue;
         float4 v = red[b][0][wave][lane];
 #pragma unroll
@@ -195,13 +192,13 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
         const float sc = a.rscale[n];
         v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
         if constexpr (GU) { // gate rows m, m + 1, then up's
-            *reinterpret_cast<float2 *>(S.y + (size_t)n * M + m) =
+            *reinterpret_cast<float2 *>(a.y + (size_t)n * M + m) =
                 make_float2(silu_mul(v.x, v.z), silu_mul(v.y, v.w));
             continue;
         }
         const bool split = a.kslices > 1;
-        float *y = split ? a.part + ((size_t)z * N + n) * M : S.y + (size_t)n * M;
-        const float *rr = !split && S.residual ? S.residual + (size_t)n * M : nullptr;
+        float *y = split ? a.part + ((size_t)z * N + n) * M : a.y + (size_t)n * M;
+        const float *rr = !split && a.residual ? a.residual + (size_t)n * M : nullptr;
         if (m + 3 < M && (M & 3) == 0) {
             if (rr) {
                 const float4 o = *reinterpret_cast<const float4 *>(rr + m);
@@ -222,8 +219,7 @@ __global__ __launch_bounds__(64 * WAVES, (occupancy<F, TB>())) void regmm_kernel
 // One format's launches (each format is its own translation unit).
 template <int F> int launch_regmm_format(const regmm::Args &a, int tb, void *stream)
 {
-    const int total = a.rtiles * a.groups;
-    const dim3 grid((total + 7) / 8 * 8, a.kslices), block(64 * regmm::WAVES);
+    const dim3 grid((a.rtiles + 7) / 8 * 8, a.kslices), block(64 * regmm::WAVES);
     hipStream_t st = (hipStream_t)stream;
     const bool gu = a.up.p0;
     if (tb == 1) {
