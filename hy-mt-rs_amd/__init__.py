@@ -645,7 +645,8 @@ class DenseDecoder:
         return self
 
     def set_prefill_rows(self, rows: int) -> None:
-        """Tokens per device pass of prefill (results do not depend on it)."""
+        """Tokens per device pass of prefill (results do not depend on it,
+        but for MoE layers of Q4_K experts: hyq_dense_set_prefill_rows)."""
         check(lib().hyq_dense_set_prefill_rows(self.handle, rows))
 
     def set_trace(self, rows: int | None) -> None:

@@ -472,7 +472,12 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
     if ((uintptr_t)x_d % 16 || (uintptr_t)y_d % 16)
         return fail(HYQ_EINVAL, "matmul: device buffers must be 16-byte aligned");
     if (batch > 65535) return fail(HYQ_EINVAL, "matmul: batch %zu exceeds 65535", batch);
-    // Q8_0 at up to 128 tokens: one register-operand launch (no K split)
+    // Q8_0 in whole 256-column sets at up to 128 tokens: few_q80_kernel (no K
+    // split), with the bits of its tiles inside the expert launches of
+    // hyq_moe_shared_experts_d. In us against the form below at 21 and 64 tokens:
+    // [2048 x 2048] 9.9 / 12.0 and 11.2 / 13.0, [2048 x 1536] 8.9 / 11.5 and 9.9
+    // / 12.5; weights of more rows would be faster there ([6144 x 2048] 15.8 /
+    // 11.9 and 18.2 / 13.3, [14336 x 4096] 47.8 / 25.4 and 53.1 / 30.1).
     const bool few = w->dtype == Q8_0 && few_q80_fits((int)w->rows, (int)w->cols, (int)batch);
     // a few tokens: weights dequantized into MFMA operands in registers
     int ks = 1;
@@ -480,7 +485,7 @@ int matmul_dev(hyq_ctx *ctx, const hyq_weight *w, const float *x_d, size_t batch
     if (reg) {
         ks = regmm_kslices((int)w->rows, (int)w->cols);
         // (both entry points take the same form: only one whose temporaries
-        // fit the fixed array)
+        // fit the fixed array, which about 250,000 columns exceed)
         const size_t need = align_up(batch * w->cols * 2, 256) + batch * 4 +
                             256 + (ks > 1 ? (size_t)ks * batch * w->rows * 4 : 0);
         if (need > HYQ_NOALLOC_SCRATCH_BYTES) reg = false;

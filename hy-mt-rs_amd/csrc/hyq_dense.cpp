@@ -15,9 +15,11 @@
 // attention-output GEMM with the residual add in its epilogue, the FFN norm,
 // the gate/up GEMM with silu(g)*u in its epilogue and the down GEMM with the
 // residual add; then the last row's output norm, the lm_head GEMV and the
-// argmax. Every row's result is independent of the other rows of its pass,
-// so the device takes up to `prefill_rows` tokens per pass (default 1024)
-// instead of the reference's 256-token chunks with identical results; the
+// argmax. Every row's result is independent of the other rows of its pass
+// and, as forms that sum in different orders are chosen by the prompt's rows, of
+// the pass's size (Q4_K expert stacks apart, whose kernels are chosen by the
+// pairs of a pass), so the device takes up to `prefill_rows` tokens per pass
+// (default 1024) instead of the reference's 256-token chunks; the
 // one case where the chunking shows is kept: a prompt of 256k + 1 tokens
 // ends with a one-token chunk, which the reference runs through the batch-1
 // arm, and so does this decoder (the decode step).

@@ -13,8 +13,10 @@
 // reduction. The gate/up form computes silu(g) * u of two rows in the same
 // wave. Batch >= 2 runs on the f32 matrix instructions (v_mfma_f32_16x16x4 /
 // 32x32x2: f32 products and sums): small outputs, such as a router's, as
-// T x T tiles whose K range is split over a workgroup's eight waves, large
-// ones as 64 x 64 tiles with K in steps of 32 through LDS.
+// T x T blocks whose K range is split over a workgroup's waves (sixteen for 16
+// x 16, eight for 32 x 32), large ones as 64 x 64 tiles with K in steps of 32
+// through LDS. The form, and with it the order of the sum, follows the weight's
+// shape and the number of rows (gemm_fv).
 #include <hip/hip_runtime.h>
 
 #include "hyq_internal.hpp"

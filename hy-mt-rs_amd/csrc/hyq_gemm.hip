@@ -1017,15 +1017,16 @@ size_t gemm_split_floats(int fmt, int M, int N, int K)
     return k > 1 ? (size_t)k * N * M : 0;
 }
 
-// K slices of Weight::matmul's batched product (hyq_matmul_d). Above one
+// K slices of a tiled product of Weight::matmul (hyq_matmul_d). Above one
 // token tile (BN rows) it is gemm_kslices, a rule on the weight's shape only.
 // A batch of at most BN token rows is one token tile, so the grid is the row
 // tiles times the slices: the largest count up to 8 that keeps that grid
 // within the 256 CUs and cuts K into whole blocks (and 64-column steps) of at
-// least 256 columns, never fewer than gemm_kslices gives. A [2048 x 2048]
-// weight at 64 tokens (the MoE shared projection) runs as 8 slices on 128
-// workgroups instead of 2 slices on 32. Token rows of batches on the same
-// side of BN get identical results.
+// least 256 columns, never fewer than gemm_kslices gives. A Q4_K [2048 x 2048]
+// weight at 100 tokens runs as 8 slices on 128 workgroups instead of 2 slices
+// on 32. So a token row has the same bits in every tiled batch on its side of BN;
+// the batches that the register-operand forms take (few_q80_fits, regmm_fits)
+// sum in those forms' orders, each the same at any batch it takes.
 int matmul_kslices(int fmt, int M, int K, int batch)
 {
     const int base = gemm_kslices(fmt, M, K);

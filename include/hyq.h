@@ -114,7 +114,7 @@ int hyq_weight_info(const hyq_weight *w, int *dtype, uint64_t *dims, int *rank);
 
 /* Weight::matmul (src/quant.rs:159-344). batch == 1 runs the int8 GEMV
  * (x quantized to Q8 as Q8::quantize_into, src/quant.rs:904-922);
- * batch > 1 runs the f16-MFMA GEMM (weights dequantized to f16 in LDS). */
+ * batch > 1 runs an f16-MFMA product (weights dequantized to f16). */
 int hyq_matmul(hyq_ctx *ctx, const hyq_weight *w, const float *x, size_t batch, float *y);
 /* Weight::gemv_qkv (src/quant.rs:658-721): one Q8 and one launch for all three. */
 int hyq_gemv_qkv(hyq_ctx *ctx, const hyq_weight *q, const hyq_weight *k, const hyq_weight *v,
@@ -405,7 +405,9 @@ int hyq_dense_forward(hyq_dense *m, int32_t token, float *logits, int32_t *next)
 int hyq_dense_prefill(hyq_dense *m, const int32_t *tokens, size_t n, float *logits,
                       int32_t *next);
 /* Tokens per device pass of hyq_dense_prefill (default 1024; 1..65536). The
- * results do not depend on it; it sets the activation memory: per row about
+ * results do not depend on it, but for MoE layers of Q4_K experts, whose
+ * products take one of two forms by a pass's rows (two f32 summation orders
+ * within the f16 path's tolerance). It sets the activation memory: per row about
  * 4*hidden + 8*(heads + kv_heads)*head_dim + 6*ffn bytes, plus 528 bytes per
  * query head and attention split. No counterpart in the reference, whose
  * chunk is fixed. */

@@ -102,10 +102,11 @@ def test_fragment_tiles_equal_row_tiles(gpu_ctx):
 
 def test_batched_rows_are_independent_of_batch(gpu_ctx):
     """Each token's output row does not depend on the other tokens of the
-    batch, for batches on the same side of one 128-token tile: above it the
-    K split is a rule on the weight's shape (here none); at or below it the
-    row tiles alone leave CUs idle and K is split in two (a 128-token tile
-    boundary and partial tiles included on both sides)."""
+    batch, for batches of the tiles on the same side of 128 tokens (a weight of
+    fewer than 1024 columns, which the register-operand products of few tokens
+    leave to them): above it the K split is a rule on the weight's shape (here
+    none); at or below it the row tiles alone leave CUs idle and K is split in
+    two (partial tiles included on both sides)."""
     rows, cols = 256, 512
     w = random_matrix(Q4_K, rows, cols, seed=3)
     x = np.random.default_rng(3).normal(0, 1, 300 * cols).astype(np.float32)
@@ -126,10 +127,11 @@ def test_batched_rows_are_independent_of_batch(gpu_ctx):
                                                    (Q2_0C, 1024, 4096, 5), (STQ1_0, 512, 2048, 128)],
                          ids=["q80_shared_64", "q4k_16", "q2c_5", "stq_128"])
 def test_matmul_few_tokens_split_k(gpu_ctx, oracle, dtype, rows, cols, batch):
-    """Batches of at most 128 tokens on weights of few row tiles run with K cut
-    into up to 8 slices (Q8_0 in whole 256-column sets takes the one-launch
-    register-operand product instead: the MoE shared projection [2048x2048]
-    at 64 tokens); parity with the oracle as every batched product."""
+    """Batches of at most 128 tokens on weights of few row tiles: the tiles with
+    K cut into up to 8 slices (STQ1_0 at 128 tokens), the register-operand
+    products at up to 64 tokens, and Q8_0's in whole 256-column sets (the MoE
+    shared projection [2048x2048] at 64 tokens); parity with the oracle as
+    every batched product."""
     _print("gemm few tokens", NAMES[dtype], rows, cols, batch)
     w = random_matrix(dtype, rows, cols, seed=rows + batch)
     x = np.random.default_rng(batch).normal(0, 1, batch * cols).astype(np.float32)
@@ -162,10 +164,10 @@ def test_q80_few_tokens(gpu_ctx, oracle, rows, cols):
 
 
 def test_batched_rows_match_across_workgroup_forms(gpu_ctx):
-    """96 row tiles at 300 tokens take the 8-wave, 256-token workgroups (a
-    grid of 192); 2 and 50 tokens take the 4-wave, 128-token ones. Every
-    element sees the same operands in the same order, so the rows agree bit
-    for bit (a 256-token tile boundary and its partial tile included)."""
+    """A weight of 96 tiles of 128 rows at 300 tokens and at 2 and 50 in the
+    shapes that each takes. Every element sees the same operands in the same
+    order, so the rows agree bit for bit (a 256-token boundary and partial
+    tiles included)."""
     rows, cols = 96 * 128, 256
     for dtype, seed in ((Q4_K, 11), (Q2_0C, 12)):
         ccols = 512 if dtype == Q2_0C else cols
