@@ -32,8 +32,8 @@
 // the same 16 of up in turns of two, so that a thread's four rows of the final
 // sum are two of each and it writes silu(g) * u. The MoE's shared experts at
 // 64 tokens (Q8_0, 2 x [1536 x 2048], then [2048 x 1536]): 15.9 and 12.7 us in
-// the LDS engine, whose grids are 48 and 32 workgroups, 12.5 and 11.6 here; the layer 151.6 ->
-// 146.3 us, at 6 tokens 98.2 -> 93.9.
+// the LDS engine, whose grids are 48 and 32 workgroups, 11.2 and 10.8 here; the
+// layer 151.6 -> 144.7 us, at 6 tokens 98.2 -> 89.9.
 //
 // Every weight is the same f16 value as in the LDS engine (one fma
 // bit-identical to the decoder, one rounding); an output's terms are summed
