@@ -733,18 +733,18 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
         if (pos[j] >= 0) slot[j] = atomicAdd(&cnt[tok[j]], 1);
     __syncthreads();
     lds_scan_1024(cnt, T, lsum);
-    for (int k = t; k <= T; k += 1024) toff[k] = cnt[k];
+    for (int k = t; k <= T; k += 1024) {
+        toff[k] = cnt[k];
+        if (k < T && cnt[k + 1] - cnt[k] > PLAN_LONG) longs[atomicAdd(&nlongs, 1)] = k;
+    }
 #pragma unroll
     for (int j = 0; j < PLAN_MID_PER; ++j)
         if (pos[j] >= 0) list[cnt[tok[j]] + slot[j]] = (uint16_t)pos[j];
+    __syncthreads();
+    const int nl = __builtin_amdgcn_readfirstlane(nlongs);
     // (tab is free: every count in it was read before the scan's barriers)
     unsigned *map = reinterpret_cast<unsigned *>(tab); // [PLAN_LONGS][PLAN_MID / 32]
     constexpr int WORDS = PLAN_MID / 32;
-    for (int k = t; k < T; k += 1024)
-        if (cnt[k + 1] - cnt[k] > PLAN_LONG) longs[atomicAdd(&nlongs, 1)] = k;
-    for (int i = t; i < PLAN_LONGS * WORDS; i += 1024) map[i] = 0;
-    __syncthreads();
-    const int nl = nlongs;
     // the row of bits of the pair's token; -1 for a short list
     auto long_row = [&](int j) {
         int r = -1;
@@ -753,6 +753,8 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
         return r;
     };
     if (nl) { // (the workgroup's test)
+        for (int i = t; i < nl * WORDS; i += 1024) map[i] = 0;
+        __syncthreads();
 #pragma unroll
         for (int j = 0; j < PLAN_MID_PER; ++j) {
             const int r = pos[j] >= 0 ? long_row(j) : -1;
@@ -782,7 +784,7 @@ __global__ __launch_bounds__(1024) void moe_plan_mid_kernel(
         if (pos[j] >= 0) {
             const int lo = cnt[tok[j]], hi = cnt[tok[j] + 1];
             int r = lo;
-            if (hi - lo > PLAN_LONG) {
+            if (nl && hi - lo > PLAN_LONG) {
                 const int word = pos[j] >> 5;
                 r += list[lo + word] + __popc(map[long_row(j) * WORDS + word] &
                                               ((1u << (pos[j] & 31)) - 1u));
